@@ -18,6 +18,7 @@
 
 #include "chol.hpp"
 #include "gemm_dev.hpp"
+#include "split.hpp"
 #include "torchsum.hpp"
 
 namespace icq {
@@ -648,7 +649,21 @@ double* dinv64_of(float* dinv, int64_t batch, int64_t n) {
 // order as with one update per block (bit-identical results).
 constexpr int64_t SUPER_NB = 1024;
 
-int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* dinv64, int* info, hipStream_t st) {
+// Where the split products (split.hpp) are taken instead of gemm_f32's, by
+// the matrix's order alone (a batch's matrices equal each one by itself):
+// - merges of segments of SPLIT_SEG and more, in matrices of more than one.
+//   The level of 1024 measured 64 us in fp32 and 99 us split at 4096 (too few
+//   128-tiles), 136 and 201 us at 12288; that of 2048 187 and 173 us at 4096,
+//   484 and 347 us at 12288.  X^T X: 63 and 85 us at 2048, 198 and 118 us at
+//   2901 (rows that are not aligned), 242 and 194 us at 4096.
+// - trailing updates of at least SPLIT_SYRK_BLOCKS blocks of rows (K = 1024,
+//   splitting included): 45 and 59 us at 853 rows, 60 and 62 us at 2048 (76
+//   and 63 us at 1976 rows, not aligned), 170 and 134 us at 4096.
+constexpr int64_t SPLIT_SEG = 2048;
+constexpr int64_t SPLIT_SYRK_BLOCKS = 15;
+
+int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* dinv64, int* info, hipStream_t st,
+          const SplitPlanes* Lp) {
     const int64_t nblk = cdiv(n, NB);
     const int64_t dstride = nblk * NB * NB;
     IC_REQUIRE(batch <= 65535, "potrf: batch too large");
@@ -715,6 +730,25 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
         if (m > 0) {
             const float* P = H + s1 * ld + s0;
             const int64_t k = s1 - s0;
+            const bool split = Lp && cdiv(m, SP_ROWS) >= SPLIT_SYRK_BLOCKS;
+            if (Lp) {
+                // the rows that this update or a merge reads
+                const int64_t r = split ? s1 : cdiv(s1, SPLIT_SEG) * SPLIT_SEG;
+                int rc = split_planes(H, n, ld, sH, r, n, s0, s1, 0, 0, *Lp, batch, PT_GEMM_CHOL, st);
+                if (rc) return rc;
+            }
+            if (split) {
+                SplitOp a;
+                a.s = *Lp;
+                a.r0 = s1 / SP_ROWS;
+                a.c0 = s0 / SP_K;
+                a.zp = Lp->stride;
+                SplitGemm g{m, m, k, -1.0f, 1, a, a, H + s1 * ld + s1, ld, sH, SplitOp{}, CMASK_LOWER, KR_FULL, batch,
+                            PT_GEMM_CHOL, (double)batch * 2.0 * dtri((double)m) * k};
+                int rc = split_gemm(g, st);
+                if (rc) return rc;
+                continue;
+            }
             GemmArgs g{m, m, k, -1.0f, 1.0f, P, ld, sH, P, ld, sH, H + s1 * ld + s1, ld, sH, 0, 1, CMASK_LOWER,
                        KR_FULL, batch, PT_GEMM_CHOL, (double)batch * 2.0 * dtri((double)m) * k};
             g.chunk_sub = 1;
@@ -800,8 +834,55 @@ static int merge_pairs(const float* L, float* X, int64_t ld, int64_t r0, int64_t
     return IC_OK;
 }
 
+// The same merge from L's planes, for segments of SPLIT_SEG and more: X11's
+// planes are there (transposed), X22's are formed here (by rows), T stays in
+// planes, and X21 is written in fp32 (a later merge's X22) and, transposed,
+// beside X11's planes.
+static int merge_pairs_split(float* X, int64_t n, int64_t ld, int64_t r0, int64_t n1, int64_t n2, int64_t count,
+                             int64_t batch, int64_t sH, const SplitWork& w, hipStream_t st) {
+    const bool pairs_batched = count > 1;
+    const int64_t gb = pairs_batched ? count : batch;
+    const int64_t outer = pairs_batched ? batch : 1;
+    const int64_t step = pairs_batched ? n1 + n2 : 0;          // rows between the pairs
+    const int64_t b0 = r0 / SP_ROWS, b1 = (r0 + n1) / SP_ROWS, n2p = cdiv(n2, SP_ROWS) * SP_ROWS;
+    SplitPlanes T = w.T;
+    T.nb = n2p / SP_K;
+    const int64_t tz = pairs_batched ? n1 / SP_ROWS * T.nb * SP_CHUNK : T.stride;
+    int rc0 = split_planes(X, n, ld, sH, r0 + n1, r0 + n1 + n2, r0 + n1, r0 + n1 + n2, 0, 1, w.XR, batch, PT_GEMM_INV,
+                           st, count, count > 1 ? n1 + n2 : 0);
+    if (rc0) return rc0;
+    for (int64_t m = 0; m < outer; ++m) {
+        const int64_t off = pairs_batched ? m : 0;
+        auto op = [&](SplitPlanes s, int64_t rb, int64_t kb) {
+            SplitOp o;
+            o.s = s;
+            o.s.p += off * s.stride;
+            o.r0 = rb;
+            o.c0 = kb * SP_PER_BLOCK;
+            o.zr = step / SP_ROWS;
+            o.zc = step / SP_K;
+            o.zp = pairs_batched ? 0 : s.stride;
+            return o;
+        };
+        SplitOp t = op(T, 0, 0);
+        t.zr = t.zc = 0;
+        t.zp = tz;
+        int rc;
+        // T = L21 X11 (k >= column: X11 is lower)
+        SplitGemm g1{n2, n1, n1, 1.0f, 0, op(w.L, b1, b0), op(w.XT, b0, b0), nullptr, 0, 0, t, CMASK_FULL, KR_FROM_J,
+                     gb, PT_GEMM_INV, (double)gb * n2 * n1 * (n1 + 1)};
+        if ((rc = split_gemm(g1, st))) return rc;
+        // X21 = -X22 T (k <= row: X22 is lower)
+        SplitGemm g2{n2, n1, n2p, -1.0f, 0, op(w.XR, b1, b1), t, X + off * sH + (r0 + n1) * ld + r0, ld,
+                     pairs_batched ? step * (ld + 1) : sH, op(w.XT, b0, b1), CMASK_FULL, KR_TO_I, gb, PT_GEMM_INV,
+                     (double)gb * n1 * n2 * (n2 + 1)};
+        if ((rc = split_gemm(g2, st))) return rc;
+    }
+    return IC_OK;
+}
+
 int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_t sH, const double* dinv64,
-          hipStream_t st) {
+          hipStream_t st, const SplitWork* w) {
     const int64_t nblk = cdiv(n, NB);
     const int64_t dstride = nblk * NB * NB;
     hipLaunchKernelGGL(put_diag_all_kernel, dim3((unsigned)nblk, (unsigned)batch), dim3(256), 0, st, X, n, ld, sH,
@@ -811,7 +892,14 @@ int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_
     std::vector<int64_t> seg;
     for (int64_t k = 0; k < nblk; ++k) seg.push_back(k * NB);
     seg.push_back(n);
+    bool split = false;   // the segments' planes exist
     while (seg.size() > 2) {
+        if (w && !split && seg[1] == SPLIT_SEG) {
+            int rc = split_planes(X, n, ld, sH, 0, seg[1], 0, seg[1], 1, 1, w->XT, batch, PT_GEMM_INV, st,
+                                  (int64_t)seg.size() - 1, seg[1]);
+            if (rc) return rc;
+            split = true;
+        }
         const int64_t nseg = (int64_t)seg.size() - 1;
         const int64_t npair = nseg / 2;
         std::vector<int64_t> next;
@@ -823,7 +911,8 @@ int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_
             while (q < npair && seg[2 * q + 1] - seg[2 * q] == n1 && seg[2 * q + 2] - seg[2 * q + 1] == n2 &&
                    seg[2 * q] - seg[2 * q - 2] == n1 + n2)
                 ++q;
-            int rc = merge_pairs(L, X, ld, r0, n1, n2, q - p, (n1 + n2) * (ld + 1), batch, sH, st);
+            int rc = split ? merge_pairs_split(X, n, ld, r0, n1, n2, q - p, batch, sH, *w, st)
+                           : merge_pairs(L, X, ld, r0, n1, n2, q - p, (n1 + n2) * (ld + 1), batch, sH, st);
             if (rc) return rc;
             p = q;
         }
@@ -839,9 +928,79 @@ int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_
 
 using namespace icq;
 
+// Split planes of `batch` inverses of order n: their bytes, and (w) their
+// places from `base` on.
+static int64_t split_bytes(int64_t batch, int64_t n, char* base, SplitWork* w) {
+    const int64_t nb = cdiv(n, SP_ROWS);
+    const int64_t tri = SP_PER_BLOCK * (nb * (nb + 1) / 2) * SP_CHUNK;
+    const int64_t rect = SP_PER_BLOCK * (nb * nb / 4 + nb) * SP_CHUNK;   // n1 n2 <= n^2 / 4, whole blocks
+    if (w) {
+        uint16_t* p = reinterpret_cast<uint16_t*>(base);
+        w->L = SplitPlanes{p, SP_LOWER, nb, tri};
+        w->XT = SplitPlanes{p + batch * tri, SP_UPPER, nb, tri};
+        w->XR = SplitPlanes{p + 2 * batch * tri, SP_LOWER, nb, tri};
+        w->T = SplitPlanes{p + 3 * batch * tri, SP_RECT, 0, rect};
+    }
+    return batch * (3 * tri + rect) * (int64_t)sizeof(uint16_t);
+}
+
+// The planes take 14 n^2 bytes beside the 8 n^2 of H and X: matrices beyond
+// SPLIT_MAX_N (60 GB of planes) are inverted without them, and a batch whose
+// planes would take more than SPLIT_MAX_BYTES one matrix after the other.
+constexpr int64_t SPLIT_MAX_N = 65536, SPLIT_MAX_BYTES = 64LL << 30;
+// Up to SPLIT_ALIGNED_N the fp32 kernels keep up where their rows are aligned
+// (a layer with a 3072 x 3072 Hessian 4.03 ms, 4.08 split); where they are not
+// they do not (2901, Cholesky method: 4.13 ms, 4.05 split).
+constexpr int64_t SPLIT_ALIGNED_N = 3072;
+static bool splits(int64_t n) {
+    return n > (n % 4 == 0 ? SPLIT_ALIGNED_N : SPLIT_SEG) && n <= SPLIT_MAX_N;
+}
+static int64_t split_batch(int64_t batch, int64_t n) {
+    return split_bytes(batch, n, nullptr, nullptr) > SPLIT_MAX_BYTES ? 1 : batch;
+}
+
 extern "C" int64_t ic_hessian_inverse_workspace_bytes(int64_t batch, int64_t n) {
     return (batch * n * n + dinv_floats(batch, n)) * (int64_t)sizeof(float) +
-           dinv_floats(batch, n) * (int64_t)sizeof(double) + 256;
+           dinv_floats(batch, n) * (int64_t)sizeof(double) + 256 +
+           (splits(n) ? split_bytes(split_batch(batch, n), n, nullptr, nullptr) + 256 : 0);
+}
+
+// `batch` damped matrices H -> their inverses (ic_hessian_inverse's methods);
+// X: batch n^2 floats.
+static int inverse(float* H, int64_t batch, int64_t n, int method, int* info, int* info2, float* X, double* dinv64,
+                   const SplitWork* w, hipStream_t st) {
+    const int64_t ld = n, sH = n * n;
+    const SplitPlanes* Lp = w ? &w->L : nullptr;
+    int rc = potrf(H, batch, n, ld, sH, dinv64, info, st, Lp);
+    if (rc) return rc;
+    rc = trtri(H, X, batch, n, ld, sH, dinv64, st, w);
+    if (rc) return rc;
+    // H^-1 (upper triangle incl. diagonal) = X^T X  -> H
+    const double flops = (double)batch * 2.0 * (double)n * (n + 1) * (n + 2) / 6.0;
+    if (w) {
+        SplitOp x;
+        x.s = w->XT;
+        x.zp = w->XT.stride;
+        SplitGemm u{n, n, cdiv(n, SP_ROWS) * SP_ROWS, 1.0f, 0, x, x, H, ld, sH, SplitOp{}, CMASK_UPPER, KR_FROM_MAXIJ,
+                    batch, PT_GEMM_INV, flops};
+        rc = split_gemm(u, st);
+    } else {
+        GemmArgs u{n, n, n, 1.0f, 0.0f, X, ld, sH, X, ld, sH, H, ld, sH, 1, 0, CMASK_UPPER, KR_FROM_MAXIJ, batch,
+                   PT_GEMM_INV, flops};
+        rc = gemm_f32(u, st);
+    }
+    if (rc) return rc;
+    if (method == 2) return IC_OK;   // the lower part keeps L: finite, never read by such callers
+    if ((rc = mirror_upper(H, batch, n, ld, sH, st))) return rc;
+    if (method == 1) {
+        // upper Cholesky factor of H^-1 (converter/gptq.py:91-110): L2 = chol(H^-1), return L2^T
+        rc = potrf(H, batch, n, ld, sH, dinv64, info2, st, Lp);
+        if (rc) return rc;
+        dim3 tb(16, 16), tg((unsigned)cdiv(n, 16), (unsigned)cdiv(n, 16), (unsigned)batch);
+        hipLaunchKernelGGL(lower_to_upper_kernel, tg, tb, 0, st, H, n, ld, sH);
+        IC_CHECK_LAUNCH();
+    }
+    return IC_OK;
 }
 
 extern "C" int ic_hessian_inverse(float* H, int64_t batch, int64_t n, float damping, int method, int* info,
@@ -852,31 +1011,22 @@ extern "C" int ic_hessian_inverse(float* H, int64_t batch, int64_t n, float damp
                "ic_hessian_inverse: method must be 0 (hinv), 1 (cholesky) or 2 (hinv, upper triangle)");
     if (n == 0 || batch == 0) return IC_OK;
     hipStream_t st = as_stream(stream);
-    const int64_t ld = n, sH = n * n;
+    const int64_t sH = n * n;
     float* X = reinterpret_cast<float*>(workspace);
     float* dinv = X + batch * sH;
     double* dinv64 = dinv64_of(dinv, batch, n);
     IC_CHECK_HIP(hipMemsetAsync(info, 0, batch * sizeof(int), st));
-    hipLaunchKernelGGL(damp_kernel, dim3((unsigned)batch), dim3(256), 0, st, H, n, ld, sH, damping);
+    hipLaunchKernelGGL(damp_kernel, dim3((unsigned)batch), dim3(256), 0, st, H, n, n, sH, damping);
     IC_CHECK_LAUNCH();
-    int rc = potrf(H, batch, n, ld, sH, dinv64, info, st);
-    if (rc) return rc;
-    rc = trtri(H, X, batch, n, ld, sH, dinv64, st);
-    if (rc) return rc;
-    // H^-1 (upper triangle incl. diagonal) = X^T X  -> H
-    GemmArgs u{n, n, n, 1.0f, 0.0f, X, ld, sH, X, ld, sH, H, ld, sH, 1, 0, CMASK_UPPER, KR_FROM_MAXIJ, batch,
-               PT_GEMM_INV, (double)batch * 2.0 * (double)n * (n + 1) * (n + 2) / 6.0};
-    rc = gemm_f32(u, st);
-    if (rc) return rc;
-    dim3 tb(16, 16), tg((unsigned)cdiv(n, 16), (unsigned)cdiv(n, 16), (unsigned)batch);
-    if (method == 2) return IC_OK;   // the lower part keeps L: finite, never read by such callers
-    if ((rc = mirror_upper(H, batch, n, ld, sH, st))) return rc;
-    if (method == 1) {
-        // upper Cholesky factor of H^-1 (converter/gptq.py:91-110): L2 = chol(H^-1), return L2^T
-        rc = potrf(H, batch, n, ld, sH, dinv64, info + batch, st);
+    if (!splits(n)) return inverse(H, batch, n, method, info, info + batch, X, dinv64, nullptr, st);
+    const uintptr_t end = reinterpret_cast<uintptr_t>(dinv64 + dinv_floats(batch, n));
+    const int64_t step = split_batch(batch, n);
+    SplitWork w;
+    split_bytes(step, n, reinterpret_cast<char*>((end + 255) & ~(uintptr_t)255), &w);
+    for (int64_t b = 0; b < batch; b += step) {
+        int rc = inverse(H + b * sH, step, n, method, info + b, info + batch + b, X + b * sH,
+                         dinv64 + dinv_floats(b, n), &w, st);
         if (rc) return rc;
-        hipLaunchKernelGGL(lower_to_upper_kernel, tg, tb, 0, st, H, n, ld, sH);
-        IC_CHECK_LAUNCH();
     }
     return IC_OK;
 }

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "gemm.hpp"
+#include "split.hpp"
 
 namespace icq {
 
@@ -15,12 +16,21 @@ double* dinv64_of(float* dinv, int64_t batch, int64_t n);
 // info[b] receives the 1-based column of the first non-positive pivot (or
 // stays as it was).  The strict upper triangle is left as it was, except in
 // the 128 x 128 diagonal blocks (zeroed).
-int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* dinv64, int* info, hipStream_t st);
+// Lp: planes for L (SP_LOWER); they then hold the blocks that trtri's split
+// merges read, and the larger trailing updates are split products.
+int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* dinv64, int* info, hipStream_t st,
+          const SplitPlanes* Lp = nullptr);
+
+// Split planes of a large inverse: L (from potrf), X^T (whole on return), X
+// by rows and the merges' intermediate products.
+struct SplitWork {
+    SplitPlanes L, XT, XR, T;
+};
 
 // X = L^-1 from potrf's L and fp64 Dinv blocks (rounded to fp32 on the
 // diagonal of X): the lower triangle of X is exact, its strict upper
 // triangle outside the diagonal blocks is scratch.
 int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_t sH, const double* dinv64,
-          hipStream_t st);
+          hipStream_t st, const SplitWork* w = nullptr);
 
 }  // namespace icq
