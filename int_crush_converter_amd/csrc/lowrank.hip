@@ -19,14 +19,13 @@
 // orth() is shifted CholeskyQR3: three passes of Y <- Y chol(Y^T Y + s I)^-T,
 // the first with s = 1e-5 tr(Y^T Y), which divides the condition number by
 // ~1/sqrt(s) so that the two plain passes see <= ~1e2 and fp32 Gram
-// matrices keep them accurate.  Every piece is an fp32-MFMA GEMM or the
+// matrices keep them accurate; steps whose basis only feeds the next one
+// leave out the third.  Every piece is an fp32-MFMA GEMM or the
 // blocked Cholesky / triangular inverse of chol.hip.
 //
-// The p x p eigenproblem is two-sided cyclic Jacobi in fp64 with the
-// round-robin ordering: one launch applies the p/2 disjoint rotations of a
-// round to A (Givens from both sides, 2 x 2 blocks, upper half mirrored so
-// A stays exactly symmetric) and to V.  Sweeps run until the off-diagonal
-// norm is below 1e-12 of the diagonal's, or 40 sweeps.
+// The p x p eigenproblem is two-sided cyclic Jacobi in fp64 by blocks of 32
+// (below).  Sweeps run until the off-diagonal norm is below 1e-12 of the
+// diagonal's, or 40 sweeps.
 #include <algorithm>
 
 #include "chol.hpp"
@@ -91,15 +90,15 @@ __global__ void sumsq_kernel(const float* x, int64_t n, double* part) {
     if (threadIdx.x == 0) part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-// T[i][i] -= rel * sqrt(sum part[0..n))  (one work-group; fixed order)
+// T[i][i] -= rel * sqrt(sum part[0..n))  (one work-group of 256; fixed order)
 __global__ void sub_frob_diag_kernel(float* T, int64_t p, const double* part, int n, double rel) {
-    __shared__ double shift;
-    if (threadIdx.x == 0) {
-        double acc = 0.0;
-        for (int i = 0; i < n; ++i) acc += part[i];
-        shift = rel * sqrt(acc);
-    }
+    __shared__ double red[4];
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) acc += part[i];
+    acc = wave_sum(acc);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
     __syncthreads();
+    const double shift = rel * sqrt(red[0] + red[1] + red[2] + red[3]);
     for (int64_t i = threadIdx.x; i < p; i += blockDim.x) T[i * p + i] = (float)((double)T[i * p + i] - shift);
 }
 
@@ -132,27 +131,49 @@ __global__ void zero_upper_kernel(float* X, int64_t p) {
     }
 }
 
-// A = fp64((T + T^T) / 2), V = I
-__global__ void jacobi_init_kernel(const float* T, int64_t p, double* A, double* V) {
-    const int64_t n = p * p;
+// ------------------------------------------------------------ Jacobi
+//
+// The p indices (padded to P, a multiple of 64, with zero rows) are taken in
+// blocks of 32; a round pairs the blocks (round-robin), each pair's 64 x 64
+// part of A is rotated in LDS by one work-group (jacobi_solve_kernel), which
+// also collects the product U of its rotations, and the rest of A and V
+// follow as fp64 MFMA products with the U (jacobi_apply_kernel).  A sweep
+// meets every pair of indices once: the first round also rotates inside the
+// blocks.  Latency-bound: the 32 rounds of rotations inside a launch are the
+// chain, 1.1 us each (their angle, then LDS traffic: 64 rows of A and of U
+// read and written).  For p = 576 a round takes 40 us to solve and 9.4 us to
+// apply, 17 rounds a sweep, 6.7 ms in 8 sweeps; a launch per round of p / 2
+// single rotations, each over all of A and V, took 8.5 us: 4600 of them, 39
+// ms, in as many sweeps.
+
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+constexpr int JB = 32, JP = 2 * JB;        // block and pair of blocks
+constexpr int JPITCH = JP + 1;             // pitch of a 64-column tile in LDS (doubles): rows and columns
+                                           // both spread over the banks
+
+// A = fp64((T + T^T) / 2) and V = I, padded to P x P: zeros and the identity.
+__global__ void jacobi_init_kernel(const float* T, int64_t p, int64_t P, double* A, double* V) {
+    const int64_t n = P * P;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
          idx += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t i = idx / p, j = idx - i * p;
-        A[idx] = 0.5 * ((double)T[i * p + j] + (double)T[j * p + i]);
+        const int64_t i = idx / P, j = idx - i * P;
+        A[idx] = i < p && j < p ? 0.5 * ((double)T[i * p + j] + (double)T[j * p + i]) : 0.0;
         V[idx] = i == j ? 1.0 : 0.0;
     }
 }
 
-// Pair P of round r (round-robin over p indices, p even): index p-1 meets r,
+// Pair k of round r (round-robin over n items, n even): item n - 1 meets r,
 // the others meet by reflection about r.  Returned ordered (a < b).
-__device__ __forceinline__ void jpair(int P, int r, int p, int& a, int& b) {
-    const int m = p - 1;
-    if (P == 0) {
+__device__ __forceinline__ void jpair(int k, int r, int n, int& a, int& b) {
+    const int m = n - 1;
+    if (k == 0) {
         a = r;
         b = m;
     } else {
-        a = (r + P) % m;
-        b = (r - P + m) % m;
+        a = r + k;
+        if (a >= m) a -= m;
+        b = r - k;
+        if (b < 0) b += m;
     }
     if (a > b) {
         const int t = a;
@@ -161,75 +182,227 @@ __device__ __forceinline__ void jpair(int P, int r, int p, int& a, int& b) {
     }
 }
 
-// Rotation annihilating A[a][b] (Golub & Van Loan, symmetric Schur 2x2):
-// J = [[c, s], [-s, c]] on (a, b), A' = J^T A J; t = tan.
-__device__ __forceinline__ void jrot(const double* A, int p, int a, int b, double& c, double& s, double& t) {
-    const double apq = A[(int64_t)a * p + b];
-    if (apq == 0.0) {
+// Row of the matrix that index i (0 .. 63) of the pair of blocks (I, J) is.
+__device__ __forceinline__ int jrow(int i, int I, int J) { return i < JB ? I * JB + i : J * JB + i - JB; }
+
+// 1 / x and 1 / sqrt(x) from the hardware estimates: two Newton steps to the
+// last bits of fp64 (half the dependent operations of the IEEE quotient and
+// root; the rotations are a serial chain).
+__device__ __forceinline__ double rcp64(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+__device__ __forceinline__ double rsq64(double x) {
+    const double h = -0.5 * x;
+    double r = __builtin_amdgcn_rsq(x);
+    r = r * fma(h * r, r, 1.5);
+    return r * fma(h * r, r, 1.5);
+}
+
+// Rotation annihilating apq (Golub & Van Loan, symmetric Schur 2x2):
+// J = [[c, s], [-s, c]] on (p, q), A' = J^T A J; t = tan, the smaller root
+// 2 apq / (d + sign(d) sqrt(d^2 + 4 apq^2)) of t^2 + (d / apq) t - 1 = 0,
+// d = aqq - app.  Below 1e-140 (the squares underflow) apq counts as zero.
+__device__ __forceinline__ void jrot(double app, double apq, double aqq, double& c, double& s, double& t) {
+    const double d = aqq - app, w = fma(d, d, 4.0 * apq * apq);
+    if (fabs(apq) < 1e-140) {
         c = 1.0;
         s = 0.0;
         t = 0.0;
         return;
     }
-    const double th = (A[(int64_t)b * p + b] - A[(int64_t)a * p + a]) / (2.0 * apq);
-    const double at = fabs(th);
-    t = at > 1e150 ? 0.5 / th : (th >= 0.0 ? 1.0 : -1.0) / (at + sqrt(th * th + 1.0));
-    c = 1.0 / sqrt(t * t + 1.0);
+    const double den = fabs(d) + w * rsq64(w);
+    t = 2.0 * apq * rcp64(den);
+    if (d < 0.0) t = -t;
+    c = rsq64(fma(t, t, 1.0));
     s = t * c;
 }
 
-// One round: Aout = J^T Ain J, Vout = Vin J.  Threads [0, np^2) handle the
-// 2x2 blocks (pair P rows, pair C columns) with P <= C and write the mirror;
-// threads [np^2, np^2 + p np) handle a row of V and a pair of its columns.
-__global__ void jacobi_round_kernel(const double* Ain, double* Aout, const double* Vin, double* Vout, int p, int r) {
-    const int np = p / 2;
-    const int64_t nA = (int64_t)np * np;
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx < nA) {
-        const int P = (int)(idx / np), C = (int)(idx - (int64_t)P * np);
-        if (P > C) return;
-        int a, b;
-        jpair(P, r, p, a, b);
-        double cp, sp, tp;
-        jrot(Ain, p, a, b, cp, sp, tp);
-        if (P == C) {
-            const double apq = Ain[(int64_t)a * p + b];
-            Aout[(int64_t)a * p + a] = Ain[(int64_t)a * p + a] - tp * apq;
-            Aout[(int64_t)b * p + b] = Ain[(int64_t)b * p + b] + tp * apq;
-            Aout[(int64_t)a * p + b] = 0.0;
-            Aout[(int64_t)b * p + a] = 0.0;
-            return;
-        }
-        int c2, d;
-        jpair(C, r, p, c2, d);
-        double cc, sc, tc;
-        jrot(Ain, p, c2, d, cc, sc, tc);
-        const double x00 = Ain[(int64_t)a * p + c2], x01 = Ain[(int64_t)a * p + d];
-        const double x10 = Ain[(int64_t)b * p + c2], x11 = Ain[(int64_t)b * p + d];
-        const double y00 = cp * x00 - sp * x10, y01 = cp * x01 - sp * x11;
-        const double y10 = sp * x00 + cp * x10, y11 = sp * x01 + cp * x11;
-        const double z00 = cc * y00 - sc * y01, z01 = sc * y00 + cc * y01;
-        const double z10 = cc * y10 - sc * y11, z11 = sc * y10 + cc * y11;
-        Aout[(int64_t)a * p + c2] = z00;
-        Aout[(int64_t)a * p + d] = z01;
-        Aout[(int64_t)b * p + c2] = z10;
-        Aout[(int64_t)b * p + d] = z11;
-        Aout[(int64_t)c2 * p + a] = z00;
-        Aout[(int64_t)d * p + a] = z01;
-        Aout[(int64_t)c2 * p + b] = z10;
-        Aout[(int64_t)d * p + b] = z11;
-        return;
+// Pair blockIdx.x of round r: its 64 x 64 part of Ain through all rotations
+// between its two blocks (full: and inside them) to Aout, and their product
+// to U[pair] (64 x 64).  Per round of 32 disjoint rotations: their angles
+// (32 threads), then the 2 x 2 blocks of pairs P < C (mirrored, so that A
+// stays exactly symmetric), the diagonal ones and U's columns.
+__global__ __launch_bounds__(1024) void jacobi_solve_kernel(const double* Ain, double* Aout, double* U, int64_t P,
+                                                           int r, int nblk, int full) {
+    __shared__ double A[JP][JPITCH], W[JP][JPITCH];
+    __shared__ double rc[JB], rs[JB], rt[JB];
+    const int t = threadIdx.x;
+    int I, J;
+    jpair(blockIdx.x, r, nblk, I, J);
+    double a0[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = (t >> 6) + 16 * u, j = t & 63;
+        a0[u] = Ain[(int64_t)jrow(i, I, J) * P + jrow(j, I, J)];
     }
-    const int64_t v = idx - nA;
-    if (v >= (int64_t)p * np) return;
-    const int row = (int)(v / np), C = (int)(v - (int64_t)row * np);
-    int a, b;
-    jpair(C, r, p, a, b);
-    double c, s, t;
-    jrot(Ain, p, a, b, c, s, t);
-    const double va = Vin[(int64_t)row * p + a], vb = Vin[(int64_t)row * p + b];
-    Vout[(int64_t)row * p + a] = c * va - s * vb;
-    Vout[(int64_t)row * p + b] = s * va + c * vb;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = (t >> 6) + 16 * u, j = t & 63;
+        A[i][j] = a0[u];
+        W[i][j] = i == j ? 1.0 : 0.0;
+    }
+    // this thread's 2 x 2 block of pairs pr < pc (t < 496)
+    int pr = 0, pc = 0;
+    {
+        int id = t;
+        while (pr < JB - 1 && id >= JB - 1 - pr) { id -= JB - 1 - pr; ++pr; }
+        pc = pr + 1 + id;
+    }
+    __syncthreads();
+    const int rounds = full ? JP - 1 : JB;
+    for (int q = 0; q < rounds; ++q) {
+        auto pair_of = [&](int k, int& a, int& b) {
+            if (full) {
+                jpair(k, q, JP, a, b);
+            } else {
+                a = k;
+                b = JB + ((k + q) & (JB - 1));
+            }
+        };
+        if (t < JB) {
+            int a, b;
+            pair_of(t, a, b);
+            jrot(A[a][a], A[a][b], A[b][b], rc[t], rs[t], rt[t]);
+        }
+        __syncthreads();
+        if (t < JB * (JB - 1) / 2) {
+            int a, b, c, d;
+            pair_of(pr, a, b);
+            pair_of(pc, c, d);
+            const double cp = rc[pr], sp = rs[pr], cc = rc[pc], sc = rs[pc];
+            const double x00 = A[a][c], x01 = A[a][d], x10 = A[b][c], x11 = A[b][d];
+            const double y00 = cp * x00 - sp * x10, y01 = cp * x01 - sp * x11;
+            const double y10 = sp * x00 + cp * x10, y11 = sp * x01 + cp * x11;
+            const double z00 = cc * y00 - sc * y01, z01 = sc * y00 + cc * y01;
+            const double z10 = cc * y10 - sc * y11, z11 = sc * y10 + cc * y11;
+            A[a][c] = A[c][a] = z00;
+            A[a][d] = A[d][a] = z01;
+            A[b][c] = A[c][b] = z10;
+            A[b][d] = A[d][b] = z11;
+        } else if (t >= 512 && t < 512 + JB) {
+            int a, b;
+            pair_of(t - 512, a, b);
+            const double apq = A[a][b], tp = rt[t - 512];
+            A[a][a] = A[a][a] - tp * apq;
+            A[b][b] = A[b][b] + tp * apq;
+            A[a][b] = A[b][a] = 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int row = (t >> 5) + 32 * u, k = t & 31;
+            int a, b;
+            pair_of(k, a, b);
+            const double c = rc[k], s = rs[k], va = W[row][a], vb = W[row][b];
+            W[row][a] = c * va - s * vb;
+            W[row][b] = s * va + c * vb;
+        }
+        __syncthreads();
+    }
+    double* Up = U + (int64_t)blockIdx.x * JP * JP;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int idx = t + 1024 * u, i = idx / JP, j = idx % JP;
+        Aout[(int64_t)jrow(i, I, J) * P + jrow(j, I, J)] = A[i][j];
+        Up[idx] = W[i][j];
+    }
+}
+
+// D += A^T-or-A times B for this wave's 16 x 32 part (rows r0, columns c0) of
+// a 32 x 64 product with K = 64: a(k, i) and b(k, j) read the operands in LDS.
+// v_mfma_f64_16x16x4_f64: A[i = l%16][k = l/16], B[k = l/16][j = l%16],
+// D[i = l/16 + 4 v][j = l%16].
+template <typename FA, typename FB>
+__device__ __forceinline__ void jmul(doublex4 (&acc)[2], FA&& a, FB&& b, int r0, int c0, int lane) {
+    const int li = lane & 15, lk = lane >> 4;
+    acc[0] = acc[1] = doublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k0 = 0; k0 < JP; k0 += 4) {
+        const double av = a(k0 + lk, r0 + li);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+            acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, b(k0 + lk, c0 + 16 * c + li), acc[c], 0, 0, 0);
+    }
+}
+
+// The rest of round r: for pairs of blocks x < y the part A[x][y] becomes
+// U_x^T A[x][y] U_y (and its mirror), and 64 rows of V times each pair's
+// columns V U.  Work-group: 32 rows of one such part (a pair's part on the
+// diagonal comes from jacobi_solve_kernel).  Blocks [0, 2 np (np - 1) / 2):
+// A; then 2 np^2: V (in place: a work-group reads only what it writes).
+__global__ __launch_bounds__(256) void jacobi_apply_kernel(const double* Ain, double* Aout, double* V, const double* U,
+                                                          int64_t P, int r, int nblk) {
+    __shared__ double S[JP][JPITCH], Ux[JP][JB + 2], Uy[JP][JPITCH], Y[JB][JPITCH];
+    const int np = nblk / 2, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int li = lane & 15, lk = lane >> 4, r0 = (wave >> 1) * 16, c0 = (wave & 1) * 32;
+    const int nA = np * (np - 1);
+    const int id = blockIdx.x;
+    const bool isA = id < nA;
+    int x, y, h;
+    if (isA) {
+        int k = id >> 1;
+        h = id & 1;
+        x = 0;
+        while (k >= np - 1 - x) { k -= np - 1 - x; ++x; }
+        y = x + 1 + k;
+    } else {
+        h = (id - nA) & 1;
+        x = ((id - nA) >> 1) / np;
+        y = ((id - nA) >> 1) - x * np;
+    }
+    int I, J, K = 0, L = 0;
+    jpair(y, r, nblk, I, J);
+    if (isA) jpair(x, r, nblk, K, L);
+    // all loads in flight before the first LDS store
+    const double* Uyp = U + (int64_t)y * JP * JP;
+    double uy[16], ux[8], sv[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) uy[u] = Uyp[t + 256 * u];
+    doublex4 acc[2];
+    if (isA) {
+        const double* Uxp = U + (int64_t)x * JP * JP;
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+            sv[u] = Ain[(int64_t)jrow((t >> 6) + 4 * u, K, L) * P + jrow(t & 63, I, J)];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) ux[u] = Uxp[((t >> 5) + 8 * u) * JP + h * JB + (t & 31)];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) S[(t >> 6) + 4 * u][t & 63] = sv[u];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) Ux[(t >> 5) + 8 * u][t & 31] = ux[u];
+    } else {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            sv[u] = V[((int64_t)x * JP + h * JB + (t >> 6) + 4 * u) * P + jrow(t & 63, I, J)];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) Y[(t >> 6) + 4 * u][t & 63] = sv[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) Uy[(t >> 6) + 4 * u][t & 63] = uy[u];
+    if (isA) {
+        __syncthreads();
+        jmul(acc, [&](int k, int i) { return Ux[k][i]; }, [&](int k, int j) { return S[k][j]; }, r0, c0, lane);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Y[r0 + lk + 4 * v][c0 + 16 * c + li] = acc[c][v];
+    }
+    __syncthreads();
+    jmul(acc, [&](int k, int i) { return Y[i][k]; }, [&](int k, int j) { return Uy[k][j]; }, r0, c0, lane);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = r0 + lk + 4 * v, col = jrow(c0 + 16 * c + li, I, J);
+            if (isA) {
+                const int row = jrow(h * JB + i, K, L);
+                Aout[(int64_t)row * P + col] = acc[c][v];
+                Aout[(int64_t)col * P + row] = acc[c][v];
+            } else {
+                V[((int64_t)x * JP + h * JB + i) * P + col] = acc[c][v];
+            }
+        }
 }
 
 // part[2 b] = off-diagonal sum of squares, part[2 b + 1] = diagonal's.
@@ -257,31 +430,52 @@ __global__ void offdiag_kernel(const double* A, int64_t p, double* part) {
     }
 }
 
+// out[0], out[1] = the sums of the pairs (one work-group of 256; fixed order)
 __global__ void finish_pairs_kernel(const double* part, int n, double* out) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double a = 0.0, b = 0.0;
-        for (int i = 0; i < n; ++i) {
-            a += part[2 * i];
-            b += part[2 * i + 1];
-        }
-        out[0] = a;
-        out[1] = b;
+    __shared__ double red[2][4];
+    double a = 0.0, b = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) {
+        a += part[2 * i];
+        b += part[2 * i + 1];
+    }
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = a;
+        red[1][threadIdx.x >> 6] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        out[0] = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+        out[1] = red[1][0] + red[1][1] + red[1][2] + red[1][3];
     }
 }
 
-// Descending order of the diagonal (ties: lower index first): eigenvalue j
-// goes to position rank(j); column j of V goes to column rank(j) of Vs.
-__global__ void ritz_sort_kernel(const double* A, const double* V, int64_t p, float* evals, float* Vs) {
-    for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < p; j += (int64_t)gridDim.x * blockDim.x) {
-        const double dj = A[j * p + j];
-        int64_t rank = 0;
-        for (int64_t i = 0; i < p; ++i) {
-            const double di = A[i * p + i];
-            rank += (di > dj || (di == dj && i < j)) ? 1 : 0;
-        }
-        evals[rank] = (float)dj;
-        for (int64_t i = 0; i < p; ++i) Vs[i * p + rank] = (float)V[i * p + j];
+// Descending order of the first p diagonal entries of A (pitch P; ties:
+// lower index first): eigenvalue j goes to position rank[j].
+__global__ __launch_bounds__(256) void ritz_rank_kernel(const double* A, int64_t p, int64_t P, float* evals,
+                                                       int* rank) {
+    __shared__ double d[256];
+    const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const double dj = j < p ? A[j * P + j] : 0.0;
+    int r = 0;
+    for (int64_t i0 = 0; i0 < p; i0 += 256) {
+        __syncthreads();
+        if (i0 + threadIdx.x < p) d[threadIdx.x] = A[(i0 + threadIdx.x) * P + i0 + threadIdx.x];
+        __syncthreads();
+        const int m = (int)std::min<int64_t>(256, p - i0);
+        for (int i = 0; i < m; ++i) r += (d[i] > dj || (d[i] == dj && i0 + i < j)) ? 1 : 0;
     }
+    if (j < p) {
+        evals[r] = (float)dj;
+        rank[j] = r;
+    }
+}
+
+// Vs[i][rank[j]] = V[i][j], p x p (a work-group per row)
+__global__ void ritz_columns_kernel(const double* V, const int* rank, int64_t p, int64_t P, float* Vs) {
+    for (int64_t j = threadIdx.x; j < p; j += blockDim.x)
+        Vs[blockIdx.x * p + rank[j]] = (float)V[blockIdx.x * P + j];
 }
 
 static int egrid_lr(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(cdiv(n, 256), 4096)); }
@@ -291,8 +485,8 @@ static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // Workspace carve-up (every piece 256-byte aligned).
 struct LrWork {
     float *Y, *Q, *G, *X, *dinv, *T, *Vs, *x, *y, *Gp;
-    double *dinv64, *A0, *A1, *V0, *V1, *part, *scal;
-    int* info;
+    double *dinv64, *A0, *A1, *V, *U, *part, *scal;
+    int *info, *rank;
 };
 
 constexpr int LR_PARTS = 1024;   // partial sums of the reductions
@@ -305,7 +499,8 @@ static size_t lr_layout(int64_t n, int64_t p, char* base, LrWork* w) {
         off += align256(bytes);
         return ptr;
     };
-    const size_t np4 = (size_t)n * p * 4, pp4 = (size_t)p * p * 4, pp8 = (size_t)p * p * 8;
+    const size_t P = (size_t)cdiv(p, JP) * JP;   // Jacobi's padded order
+    const size_t np4 = (size_t)n * p * 4, pp4 = (size_t)p * p * 4, pp8 = P * P * 8;
     LrWork t{};
     t.Y = (float*)take(np4);
     t.Q = (float*)take(np4);
@@ -319,8 +514,9 @@ static size_t lr_layout(int64_t n, int64_t p, char* base, LrWork* w) {
     t.dinv = (float*)take((size_t)dinv_floats(1, p) * 4 + (size_t)dinv_floats(1, p) * 8 + 512);
     t.A0 = (double*)take(pp8);
     t.A1 = (double*)take(pp8);
-    t.V0 = (double*)take(pp8);
-    t.V1 = (double*)take(pp8);
+    t.V = (double*)take(pp8);
+    t.U = (double*)take(P / JP * JP * JP * 8);
+    t.rank = (int*)take((size_t)p * 4);
     t.part = (double*)take((size_t)LR_PARTS * 2 * 8);
     t.scal = (double*)take(8 * 8);
     t.info = (int*)take(64);
@@ -381,22 +577,21 @@ static int cholqr_pass(const float* Y, float* Q, int64_t n, int64_t p, float shi
     return gemm_f32(q, st);
 }
 
-// Shifted CholeskyQR3 of Y (overwritten) into Q; `well_conditioned` (a
-// Gaussian start, cond ~ (1 + sqrt(p/n)) / (1 - sqrt(p/n))) skips the
-// shifted pass: plain CholeskyQR2.
-static int orth(float* Y, float* Q, int64_t n, int64_t p, const LrWork& w, hipStream_t st,
-                bool well_conditioned = false) {
-    int rc;
-    if (well_conditioned) {
-        rc = cholqr_pass(Y, Q, n, p, 0.0f, w, st);
-        if (!rc) rc = cholqr_pass(Q, Y, n, p, 0.0f, w, st);
-        if (!rc) IC_CHECK_HIP(hipMemcpyAsync(Q, Y, (size_t)n * p * sizeof(float), hipMemcpyDeviceToDevice, st));
-        return rc;
+// Orthonormal basis of the columns of w.Y into w.Q (the two buffers trade
+// places as needed; Y's content is lost).  ORTH_START: a Gaussian start
+// (cond ~ (1 + sqrt(p/n)) / (1 - sqrt(p/n))), two plain passes.  ORTH_FULL:
+// shifted CholeskyQR3.  ORTH_STEP: its first two passes - the shifted one
+// leaves a condition number of about 10 and the second an error of about
+// 1e-5, where the next product with (H + mu I) only needs a well-conditioned
+// basis of the same space.
+enum Orth { ORTH_START, ORTH_STEP, ORTH_FULL };
+static int orth(LrWork& w, int64_t n, int64_t p, Orth kind, hipStream_t st) {
+    for (int pass = 0; pass < (kind == ORTH_FULL ? 3 : 2); ++pass) {
+        if (pass) std::swap(w.Y, w.Q);
+        int rc = cholqr_pass(w.Y, w.Q, n, p, pass == 0 && kind != ORTH_START ? 1e-5f : 0.0f, w, st);
+        if (rc) return rc;
     }
-    rc = cholqr_pass(Y, Q, n, p, 1e-5f, w, st);
-    if (!rc) rc = cholqr_pass(Q, Y, n, p, 0.0f, w, st);
-    if (!rc) rc = cholqr_pass(Y, Q, n, p, 0.0f, w, st);
-    return rc;
+    return IC_OK;
 }
 
 constexpr int JACOBI_MAX_SWEEPS = 40;
@@ -437,7 +632,7 @@ extern "C" int ic_lowrank_eigs(const float* H, int64_t n, int64_t p, int iters, 
     }
     hipLaunchKernelGGL(randn_kernel, dim3(egrid_lr(np)), dim3(256), 0, st, w.Y, np, (uint64_t)seed);
     IC_CHECK_LAUNCH();
-    int rc = orth(w.Y, w.Q, n, p, w, st, /*well_conditioned=*/true);
+    int rc = orth(w, n, p, ORTH_START, st);
     if (rc) return rc;
     // the refusal certificate is tried after one and after two steps (the
     // random start's Ritz values sit near the mean eigenvalue; one step of
@@ -470,7 +665,9 @@ extern "C" int ic_lowrank_eigs(const float* H, int64_t n, int64_t p, int iters, 
         if (it == iters) break;
         hipLaunchKernelGGL(axpy_dev_kernel, dim3(egrid_lr(np)), dim3(256), 0, st, w.Y, w.Q, np, w.scal);
         IC_CHECK_LAUNCH();
-        if ((rc = orth(w.Y, w.Q, n, p, w, st))) return rc;
+        // the certificate and the Rayleigh-Ritz step want an orthonormal basis
+        const bool full = it + 1 == iters || (it + 1 >= test_lo && it + 1 <= test_hi);
+        if ((rc = orth(w, n, p, full ? ORTH_FULL : ORTH_STEP, st))) return rc;
     }
     // Rayleigh-Ritz: T = Q^T (H Q)
     if ((rc = gram(w.Q, w.Y, n, p, w.T, w, CMASK_FULL, st))) return rc;
@@ -478,31 +675,36 @@ extern "C" int ic_lowrank_eigs(const float* H, int64_t n, int64_t p, int iters, 
     IC_CHECK_HIP(hipMemcpyAsync(&info, w.info, sizeof(int), hipMemcpyDeviceToHost, st));
     IC_CHECK_HIP(hipStreamSynchronize(st));
     if (info != 0) return fail(IC_ERR_RANGE, "ic_lowrank_eigs: orthonormalisation lost positive definiteness");
-    hipLaunchKernelGGL(jacobi_init_kernel, dim3(egrid_lr(p * p)), dim3(256), 0, st, w.T, p, w.A0, w.V0);
+    const int64_t P = cdiv(p, JP) * JP;
+    const int nblk = (int)(P / JB), npair = nblk / 2;
+    hipLaunchKernelGGL(jacobi_init_kernel, dim3(egrid_lr(P * P)), dim3(256), 0, st, w.T, p, P, w.A0, w.V);
     IC_CHECK_LAUNCH();
-    double *A = w.A0, *An = w.A1, *V = w.V0, *Vn = w.V1;
-    const int64_t threads = (p / 2) * (p / 2) + p * (p / 2);
-    const unsigned blocks = (unsigned)cdiv(threads, 256);
-    const int off_blocks = (int)std::min<int64_t>(LR_PARTS, cdiv(p * p, 256));
+    double *A = w.A0, *An = w.A1;
+    const unsigned apply = (unsigned)(npair * (npair - 1) + 2 * npair * npair);
+    const int off_blocks = (int)std::min<int64_t>(LR_PARTS, cdiv(P * P, 256));
     int sweeps = 0;
     for (; sweeps < JACOBI_MAX_SWEEPS; ++sweeps) {
-        hipLaunchKernelGGL(offdiag_kernel, dim3(off_blocks), dim3(256), 0, st, A, p, w.part);
+        hipLaunchKernelGGL(offdiag_kernel, dim3(off_blocks), dim3(256), 0, st, A, P, w.part);
         IC_CHECK_LAUNCH();
-        hipLaunchKernelGGL(finish_pairs_kernel, dim3(1), dim3(64), 0, st, w.part, off_blocks, w.scal + 2);
+        hipLaunchKernelGGL(finish_pairs_kernel, dim3(1), dim3(256), 0, st, w.part, off_blocks, w.scal + 2);
         IC_CHECK_LAUNCH();
         double od[2];
         IC_CHECK_HIP(hipMemcpyAsync(od, w.scal + 2, sizeof(od), hipMemcpyDeviceToHost, st));
         IC_CHECK_HIP(hipStreamSynchronize(st));
         if (!(od[0] > 1e-24 * od[1])) break;   // converged (or NaN: the caller sees NaN eigenvalues)
-        for (int r = 0; r < p - 1; ++r) {
-            hipLaunchKernelGGL(jacobi_round_kernel, dim3(blocks), dim3(256), 0, st, A, An, V, Vn, (int)p, r);
+        for (int r = 0; r < nblk - 1; ++r) {
+            hipLaunchKernelGGL(jacobi_solve_kernel, dim3(npair), dim3(1024), 0, st, A, An, w.U, P, r, nblk,
+                               r == 0 ? 1 : 0);
+            IC_CHECK_LAUNCH();
+            hipLaunchKernelGGL(jacobi_apply_kernel, dim3(apply), dim3(256), 0, st, A, An, w.V, w.U, P, r, nblk);
             IC_CHECK_LAUNCH();
             std::swap(A, An);
-            std::swap(V, Vn);
         }
     }
     if (sweeps_out) *sweeps_out = sweeps;
-    hipLaunchKernelGGL(ritz_sort_kernel, dim3((unsigned)cdiv(p, 64)), dim3(64), 0, st, A, V, p, evals, w.Vs);
+    hipLaunchKernelGGL(ritz_rank_kernel, dim3((unsigned)cdiv(p, 256)), dim3(256), 0, st, A, p, P, evals, w.rank);
+    IC_CHECK_LAUNCH();
+    hipLaunchKernelGGL(ritz_columns_kernel, dim3((unsigned)p), dim3(256), 0, st, w.V, w.rank, p, P, w.Vs);
     IC_CHECK_LAUNCH();
     // eigenvectors of H: Q Vs
     GemmArgs e{n, p, p, 1.0f, 0.0f, w.Q, p, 0, w.Vs, p, 0, evecs, p, 0, 0, 0, CMASK_FULL, KR_FULL, 1, PT_OTHER};
