@@ -5,11 +5,12 @@
 //
 //  1. damp:   H += fp32(damping) * max(mean(diag H), 1e-6) * I   (per matrix)
 //  2. potrf:  blocked right-looking Cholesky, nb = 128.  The nb x nb diagonal
-//             block is factored in LDS by one workgroup, which also writes
-//             its triangular inverse Dinv_k; the panel is A21 <- A21 Dinv_k^T
-//             and the trailing update A22 -= A21 A21^T, both fp32-MFMA GEMMs.
-//  3. trtri:  X = L^-1: diagonal blocks Dinv_k, then adjacent diagonal
-//             inverses merged level by level, X21 = -X22 (L21 X11)  (GEMMs)
+//             block is factored by one work-group, the panel is solved with
+//             it (both fp64), and the trailing update A22 -= A21 A21^T is a
+//             GEMM.
+//  3. trtri:  X = L^-1: the diagonal blocks' inverses (fp64), then adjacent
+//             diagonal inverses merged level by level, X21 = -X22 (L21 X11)
+//             (GEMMs)
 //  4. lauum:  H^-1 (upper triangle) = X^T X, one GEMM whose tile (I, J)
 //             only runs k >= max(I, J) because X is lower triangular.
 // Flops: n^3/3 each for 2-4; all but the nb x nb factorisations are MFMA.
@@ -81,46 +82,43 @@ __global__ __launch_bounds__(256) void damp_kernel(float* H, int64_t n, int64_t 
     }
 }
 
-// Factor the diagonal block [k0, k0+nb) of matrix blockIdx.x in place (lower,
-// upper part of the block set to 0) and write Dinv = L_kk^-1 (lower, upper 0)
-// to dinv64 (fp64, pitch NB).  info[b] gets the
-// 1-based column of the first non-positive pivot (LAPACK convention) if it
-// is still 0.  A partial block (nb < 128) is padded with the identity.
+// Factor the diagonal block [k0, k0+nb) of a matrix in place (lower, upper
+// part of the block set to 0) and write what the panel solve and the
+// triangular inverse need of it to dinv64 (packed tiles, below).  info[b]
+// gets the 1-based column of the first non-positive pivot (LAPACK convention)
+// if it is still 0.  A partial block (nb < 128) is padded with the identity.
 //
-// The arithmetic is fp64 (inputs and outputs fp32 / fp64): the diagonal
-// blocks and their inverses feed every later step, and an fp64 factor keeps
-// the whole inverse at the accuracy of the reference's LAPACK fp32 path.
+// The arithmetic is fp64 (inputs and outputs fp32): the diagonal blocks feed
+// every later step, and an fp64 factor and panel solve keep the whole inverse
+// at the accuracy of the reference's LAPACK fp32 path.
 //
-// The block is processed in 16 panels of 8 columns by 8 waves.  Both the
-// block A and R (X = L^-1 under construction, started as I) live in MFMA
-// accumulators: the 36 lower 16x16 tiles of each are dealt to waves 1..7
-// round-robin in column-major order (so one tile column spreads over
-// several waves).  Wave 0 owns no tile: it runs the serial part, the
-// column-by-column factorisation of each panel and the forward substitution
-// for the rows of X, while the other waves apply the rank-8 updates on the
-// matrix cores (v_mfma_f64_16x16x4_f64).  Look-ahead keeps the factorisation
-// off the MFMA path; iteration it has two phases:
-//   U: wave 0 factors panel it (from the published tile column, two rows
-//      per lane, pivots and the panel's rows broadcast by readlane); the
-//      others apply panel it - 1's update A -= L L^T to every live tile
-//      outside the next tile column (which got it in phase A of it - 1) and
-//      panel it - 2's update R -= L X to R, then publish rows of R of panel
-//      it - 1 (now final up to their own diagonal block);
-//   A: the owners of the tile column holding panel it + 1 apply panel it's
-//      update to it and publish it for wave 0; waves 0 and 1 turn the
-//      published rows of R into the rows of X of panel it - 1 (forward
-//      substitution with that panel's 8x8 diagonal block, a column per
-//      lane) and store them to Dinv / Dinv64 (whole rows: coalesced).
-// Every element receives its updates in panel order with the same fp64
-// operations, so the result does not depend on the schedule.  Elements that
-// are already final (or above the diagonal) may receive updates; they are
-// never read again.  At the end the block writes the image of L row by row.
+// Bound by the serial chain of 128 columns on one CU.  The block is processed
+// in 8 panels of 16 columns: wave 0 factors and inverts the diagonal
+// tiles, six other waves (W = 1..6) own the other 16x16 tiles of the lower triangle
+// (in MFMA accumulators, dealt round-robin in column-major order, so that a
+// tile column has one tile per wave, the first one of a wave two).  Panel J has two phases:
+//   F: wave 0 updates its copy of tile (J, J) with panel J - 1 and factors
+//      it; the others apply panel J - 1's update A -= L L^T to their tiles of
+//      columns >= J, hand tile (J + 1, J + 1) to wave 0 and write panel J - 1;
+//   S: the owners of the tiles below it solve L_IJ^T = L_JJ^-1 A_IJ^T.
+// Tiles are held transposed, so that a solved fragment (D layout) is at once
+// the operand of the updates (v_mfma_f64_16x16x4_f64 throughout).  Every
+// element receives its updates in panel order with the same fp64 operations,
+// so the result does not depend on the schedule.
 //
 // MFMA 16x16x4 f64 operand layout (lane l of 64; D differs from the f32
 // variant's 4*(l/16) + v):
 //   A: A[i = l%16][k = l/16]      B: B[k = l/16][j = l%16]
 //   D (4 doubles v): D[i = l/16 + 4*v][j = l%16]
+// so a D fragment is the B operand of four MFMA steps as it stands.
+//
+// Packed tiles: tile (J, K), K <= J, of a block's factor at dinv64 +
+// (J (J + 1) / 2 + K) * 256, in A-operand order with two steps adjacent:
+// value [h][lane][e] is L[16 J + perm16(l%16)][16 K + 4 (l/16) + 2 h + e], and on the
+// diagonal the same of L_JJ^-1.  perm16 orders the 16 indices so that the four
+// that a lane's D fragment holds are adjacent in memory (4 g .. 4 g + 3).
 typedef double ddoublex4 __attribute__((ext_vector_type(4)));
+typedef double ddoublex2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ double rdlane(double v, int l) {
     const int64_t b = __double_as_longlong(v);
@@ -129,12 +127,20 @@ __device__ __forceinline__ double rdlane(double v, int l) {
     return __longlong_as_double(((int64_t)hi << 32) | (uint32_t)lo);
 }
 
-constexpr int DIAG_WAVES = 8;            // wave 0: factorisation; 1..7: tiles
-constexpr int DIAG_TILES = 36;           // lower 16x16 tiles of the 8x8 tile grid
+// Work-group: wave 0 factors; waves 1, 2, 3, 5, 6, 7 hold tiles.  Wave 4 only
+// helps to stage: it shares wave 0's SIMD, where another wave's fp64 MFMAs
+// would hold its chain up (fp64 vector and matrix instructions share a unit).
+constexpr int DIAG_WAVES = 8, TILE_WAVES = 6;
+constexpr int DT = 16, DN = NB / DT;     // tile, tiles per side
+constexpr int DIAG_TILES = DN * (DN + 1) / 2;
 constexpr int DSLOTS = 6;                // tiles per MFMA wave (at most)
+constexpr int64_t PACKED = DT * DT;      // doubles of a packed tile
+
+__host__ __device__ constexpr int packed_at(int J, int K) { return J * (J + 1) / 2 + K; }
+__device__ __forceinline__ constexpr int perm16(int i) { return 4 * (i & 3) + (i >> 2); }
 
 // Lower tile `id` in column-major order over the lower triangle: tile column
-// and tile row.  Wave W (1..7) owns the tiles id = W - 1 + 7 s.
+// and tile row.  Tile wave W (1..6) owns the tiles id = W - 1 + 6 s.
 constexpr int cm_col(int id) {
     int J = 0;
     while (id >= 8 - J) { id -= 8 - J; ++J; }
@@ -145,7 +151,7 @@ constexpr int cm_row(int id) {
     while (id >= 8 - J) { id -= 8 - J; ++J; }
     return J + id;
 }
-constexpr int tile_id(int W, int s) { return W - 1 + 7 * s; }
+constexpr int tile_id(int W, int s) { return W - 1 + TILE_WAVES * s; }
 
 // Slot S of wave W as compile-time constants, and a loop over a wave's
 // slots that hands each one to f as a type (so every tile coordinate is a
@@ -166,306 +172,311 @@ __device__ __forceinline__ void each_slot(F&& f) {
     each_slot_impl<W>(f, std::make_integer_sequence<int, DSLOTS>{});
 }
 
-// Panel-local k (0..7) is stored at kperm(k), so that the two k values a
-// lane feeds to the two MFMA steps of a panel, lr and lr + 4, are adjacent.
-__device__ __forceinline__ constexpr int kperm(int k) { return (k & 3) * 2 + (k >> 2); }
-
-// Rows of 8 doubles are padded to DP = 9, so that a wave's 64 row-wise
-// accesses spread over the LDS banks (a 64-byte pitch would put them on 4).
-// Arrays indexed by a row of the block have a spare row NB, where accesses
-// for rows past the block are clamped (so they need no branch).
-constexpr int DP = 9, RP = 17;
-constexpr int PLBUF = 3;   // L panels in use: it (phase A), it - 1 (A update), it - 2 (R update)
+constexpr int IP = DT + 1;   // pitch of the inverse tile
+constexpr int UP = NB + 4;   // pitch of the staged panel rows of the block's update
 
 struct DiagShared {
-    double pRaw[NB + 1][RP];       // the tile column of A holding the next panel (row NB stays 0)
-    double pL[PLBUF][NB + 1][DP];  // final L columns of the last three panels, at kperm
-    double dL[2][8][8];            // the 8x8 diagonal blocks of L of the last two panels
-    double rinv[2][8];             // and their pivots' reciprocal square roots
-    double rowR[8][NB];            // rows of R of the panel whose X rows are due
-    double rowXt[NB][DP];          // final rows of X = L^-1 of that panel, transposed, at kperm
-    float Lfin[NB + 1][NB + 1];    // L as it is finalised (on and below the diagonal)
+    union {
+        float P[NB * UP];         // the previous block's panel rows that update this block
+        double op[DN][4][64];     // the last panel's L_IJ, operand form: [step][lane]; over the first 32 rows of
+    };                            // P, which only the updates of tile columns 0 and 1 read (before the first L_IJ)
+    double dg[4][64];             // the next diagonal tile, D layout
+    double inv[DT][IP];           // L_JJ^-1
 };
+static_assert(sizeof(double) * DN * 4 * 64 <= sizeof(float) * 2 * DT * UP, "the panel's operands fit");
 
-// The phases of the diagonal-block kernel hand data to each other only
-// through LDS, so they are separated by lds_barrier() (common.hpp), which
-// does not wait for the global stores of the Dinv rows.
+// The phases hand data to each other only through LDS, so they are separated
+// by lds_barrier() (common.hpp), which does not wait for global stores.
 
-// Rows 8 p .. 8 p + 7 of X = L^-1, column q: forward substitution with panel
-// p's 8x8 diagonal block of L from the published rows of R; the result goes
-// to rowXt (for the R updates) and to Dinv64 (whole rows: coalesced over the
-// lanes).  Phase A splits the columns over waves 0 and 1.
-__device__ __forceinline__ void x_rows(DiagShared& sh, int p, int q, int nb, double* D64) {
-    const int x0 = p * 8, xb = p & 1;
-    double x[8], l[8][8], ri[8];
+// Wave 0: the Cholesky factor of the symmetric tile `acc` (D layout), as
+// Lt = L^T, and X = L^-1, by rank-1 updates on the matrix cores: row c of the
+// tile, scaled, is an MFMA operand where it stands (its lanes are those of one
+// k), so neither the update nor the elimination of the identity needs a
+// broadcast; only the pivot goes through readlane.  A column takes about 170
+// cycles (420 with the panel's rows broadcast by readlane, 26 of 31 us a
+// block).  col0: the tile's first column, for `bad`.
+__device__ __forceinline__ void factor_tile(ddoublex4& acc, ddoublex4& Lt, ddoublex4& X, int lane, int col0,
+                                            int& bad) {
+    const int lr = lane >> 4, lj = lane & 15;
+    ddoublex4 R;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        x[c] = sh.rowR[c][q];
-        ri[c] = sh.rinv[xb][c];
-#pragma unroll
-        for (int c2 = 0; c2 < c; ++c2) l[c][c2] = sh.dL[xb][c][c2];
+    for (int v = 0; v < 4; ++v) {
+        R[v] = lr + 4 * v == lj ? 1.0 : 0.0;
+        Lt[v] = X[v] = 0.0;
     }
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-#pragma unroll
-        for (int c2 = 0; c2 < c; ++c2) x[c] = fma(-l[c][c2], x[c2], x[c]);
-        x[c] = q <= x0 + 7 ? x[c] * ri[c] : 0.0;
-    }
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        sh.rowXt[q][kperm(c)] = x[c];
-        const int row = x0 + c;
-        D64[row * NB + q] = (row < nb && q < nb) ? x[c] : 0.0;
-    }
-}
-
-// Panel it (columns j0 .. j0 + 7, rows j0 .. 127) on wave 0, two rows per
-// lane: rows j0 + lane and (TWO: it < 8) j0 + 64 + lane.  From it = 8 on
-// the second set lies past the block and is skipped.  Pivots and the
-// panel's rows are broadcast by readlane.
-template <bool TWO>
-__device__ __forceinline__ void factor_panel(DiagShared& sh, int it, int lane, int& bad) {
-    const int j0 = it * 8, co = (it & 1) * 8, pb = it % PLBUF, db = it & 1;
-    // rows past the block read the zero row NB
-    const int ra = j0 + lane, rb = j0 + lane + 64;
-    const int rac = ra < NB ? ra : NB, rbc = rb < NB ? rb : NB;
-    double va[8], vb[8], rinvv[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        va[c] = sh.pRaw[rac][co + c];
-        vb[c] = TWO ? sh.pRaw[rbc][co + c] : 0.0;
-    }
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        double d = rdlane(va[c], c);
-        if (!(d > 0.0)) {
-            if (!bad) bad = j0 + c + 1;
-            d = 1.0;
+    double pn = 0.0, prinv = 0.0;   // the previous column's -l and 1 / sqrt(pivot)
+    auto column = [&](auto cc) {
+        constexpr int c = decltype(cc)::value, v = c >> 2, g = c & 3;
+        const double r = acc[v];
+        const double d = rdlane(r, 16 * g + c);
+        double r0 = __builtin_amdgcn_rsq(d);
+        __builtin_amdgcn_sched_barrier(0);
+        // the previous column's elimination of the identity, behind the root
+        if constexpr (c > 0) {
+            constexpr int w = (c - 1) >> 2;
+            const bool row = lr == ((c - 1) & 3);
+            const double x = (row ? R[w] : 0.0) * prinv;
+            X[w] = row ? x : X[w];
+            R = __builtin_amdgcn_mfma_f64_16x16x4f64(pn, x, R, 0, 0, 0);
         }
-        // 1/sqrt(d) from the hardware estimate and two Newton steps
-        // (relative error far below fp32's), then sqrt(d) = d / sqrt(d)
-        double rinv = __builtin_amdgcn_rsq(d);
-        rinv = rinv * fma(-0.5 * d * rinv, rinv, 1.5);
-        rinv = rinv * fma(-0.5 * d * rinv, rinv, 1.5);
-        const double ljj = d * rinv;
-        va[c] = lane > c ? va[c] * rinv : (lane == c ? ljj : 0.0);
-        if (TWO) vb[c] = vb[c] * rinv;
-        rinvv[c] = rinv;
+        __builtin_amdgcn_sched_barrier(0);
+        // l = r / sqrt(d): the hardware estimate r0 of 1/sqrt(d) (relative
+        // error e/2) and one step of third order, r0 (1 + e/2 + 3/8 e^2),
+        // applied to r r0; a bad pivot's root counts as 1
+        const bool ok = d > 0.0;
+        r0 = ok ? r0 : 1.0;
+        const double rm = lr == g && lj >= c ? r : 0.0;
+        double rn = -rm;
+        asm volatile("" : "+v"(rn));   // l and -l side by side, not one after the other
+        const double q = rm * r0, qn = rn * r0;
+        double e = fma(-d * r0, r0, 1.0);
+        e = ok ? e : 0.0;
+        const double ep = e * fma(0.375, e, 0.5);
+        const double l = fma(q, ep, q), nl = fma(qn, ep, qn);
+        // (row and column c, finished, become rounding errors)
+        if constexpr (c < DT - 1) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(nl, l, acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        bad = !ok && !bad ? col0 + c + 1 : bad;
+        Lt[v] = lr == g ? l : Lt[v];
+        pn = nl;
+        prinv = fma(r0, ep, r0);
+    };
+    static_for<0, DT>(column);
+    X[3] = lr == 3 ? R[3] * prinv : X[3];   // the last row
+}
+
+// Rows of tile (I, J) of the block from memory into D layout, transposed
+// (element (row lr + 4 v of J, column lj of I) is C[16 I + lj][16 J + lr + 4 v];
+// a diagonal tile is symmetric, its upper part taken from the lower), loads
+// clamped into the block (no branch); outside it the identity.
+__device__ __forceinline__ void load_tile(const float* A, int64_t ld, int nb, int I, int J, int lr, int lj,
+                                          float (&raw)[4]) {
 #pragma unroll
-        for (int c2 = c + 1; c2 < 8; ++c2) {
-            const double lk = rdlane(va[c], c2);
-            va[c2] = fma(-va[c], lk, va[c2]);
-            if (TWO) vb[c2] = fma(-vb[c], lk, vb[c2]);
+    for (int v = 0; v < 4; ++v) {
+        int i = I * DT + lj, j = J * DT + lr + 4 * v;
+        if (I == J && i < j) {
+            const int t = i;
+            i = j;
+            j = t;
         }
-    }
-    // the panel's L columns (fp64 MFMA operands), its 8x8 diagonal block and
-    // pivots for the rows of X, and the fp32 image of L (rows past the block
-    // go to the spare row NB).  Rows of pL above the panel keep older values:
-    // they only reach elements that are final already, which are never read
-    // again.
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        sh.pL[pb][rac][kperm(c)] = va[c];
-        sh.Lfin[rac][j0 + c] = (float)va[c];
-        if (TWO) {
-            sh.pL[pb][rbc][kperm(c)] = vb[c];
-            sh.Lfin[rbc][j0 + c] = (float)vb[c];
-        }
-    }
-    if (lane < 8) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) sh.dL[db][lane][c] = va[c];
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) sh.rinv[db][c] = rinvv[c];
+        const int ic = i < nb ? i : nb - 1, jc = j < nb ? j : nb - 1;
+        const float x = A[(int64_t)ic * ld + jc];
+        raw[v] = i < nb ? x : (i == j ? 1.0f : 0.0f);
     }
 }
 
-// Wave 0: phase U factors panel it, phase A finishes columns 0..63 of the
-// rows of X of panel it - 1.  Two barriers per iteration, matching
-// diag_tile_wave.
-__device__ __forceinline__ void diag_factor_wave(DiagShared& sh, int nb, double* D64, int lane, int& bad) {
-    for (int it = 0; it <= 16; ++it) {
-        if (it < 8) factor_panel<true>(sh, it, lane, bad);
-        else if (it < 16) factor_panel<false>(sh, it, lane, bad);
-        lds_barrier();
-        if (it >= 1) x_rows(sh, it - 1, lane, nb, D64);
-        lds_barrier();
+// The same tile of P P^T (P: the staged panel rows), fp32 products as in the
+// update of the columns beside the block; added to the tile negated.  k = 16 q
+// + 4 lr + s in step s: one 16-byte read per operand and four steps; the A
+// operand's rows are taken in perm16 order, so that the f32 result (row
+// 4 (l/16) + v) has the f64 accumulators' rows.
+__device__ __forceinline__ void tile_update(const float* P, int I, int J, int lr, int lj, ddoublex4& acc) {
+    gk::floatx4 u[2];
+    u[0] = u[1] = gk::floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < NB / 16; ++q) {
+        const gk::floatx4 a = *reinterpret_cast<const gk::floatx4*>(&P[(J * DT + perm16(lj)) * UP + 16 * q + 4 * lr]);
+        const gk::floatx4 b = *reinterpret_cast<const gk::floatx4*>(&P[(I * DT + lj) * UP + 16 * q + 4 * lr]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) u[s & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], u[s & 1], 0, 0, 0);
     }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] -= (double)u[0][v] + (double)u[1][v];
 }
 
-// Operands of a rank-8 update from an L panel (or the X rows) in LDS:
-// op[r][ks] = P[16 r + lj][2 lr + ks] (panel columns 4 ks + lr, at kperm).
-__device__ __forceinline__ void load_op(const double (*P)[DP], int r, int lr, int lj, double (&op)[2]) {
-    op[0] = P[r * 16 + lj][2 * lr];
-    op[1] = P[r * 16 + lj][2 * lr + 1];
-}
-
-// Waves 1..7: the tiles of A and R.  Every tile coordinate is a compile-time
-// constant, so accumulators are indexed statically.
-template <int W>
-__device__ __forceinline__ void diag_tile_wave(DiagShared& sh, const float* A, int64_t ld, int nb, double* D64,
+// Tile wave W: the tiles below the diagonal, and the diagonal ones until they
+// go to wave 0 (tile (0, 0) is there from the start).  UPD: P P^T is
+// subtracted first, tile column J + 1 in phase F of panel J.
+template <int W, bool UPD>
+__device__ __forceinline__ void diag_tile_wave(DiagShared& sh, float* A, int64_t ld, int nb, double* packed,
                                                int lane) {
-    const int lr = lane >> 4, lj = lane & 15;   // accumulator v holds row lr + 4 v, column lj
-    ddoublex4 accA[DSLOTS], accX[DSLOTS];
-    // all loads in flight at once: addresses are clamped into the block (no
-    // branch) and values outside it replaced
+    const int lr = lane >> 4, lj = lane & 15;
+    ddoublex4 acc[DSLOTS];
     float raw[DSLOTS][4];
     each_slot<W>([&](auto t) {
         using T = decltype(t);
-        if constexpr (T::ok) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = T::I * 16 + lr + 4 * v, j = T::J * 16 + lj;
-                const int ic = i < nb ? i : nb - 1, jc = j < nb ? j : nb - 1;
-                raw[T::s][v] = A[(int64_t)ic * ld + jc];
-            }
-        }
+        if constexpr (T::ok && T::I + T::J > 0) load_tile(A, ld, nb, T::I, T::J, lr, lj, raw[T::s]);
     });
+    if (UPD) __syncthreads();   // sh.P
     each_slot<W>([&](auto t) {
         using T = decltype(t);
-        if constexpr (T::ok) {
+        if constexpr (T::ok && T::I + T::J > 0) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = T::I * 16 + lr + 4 * v, j = T::J * 16 + lj;
-                const double pad = (i == j) ? 1.0 : 0.0;
-                accA[T::s][v] = j > i ? 0.0 : (i < nb ? (double)raw[T::s][v] : pad);
-                accX[T::s][v] = pad;
-            }
+            for (int v = 0; v < 4; ++v) acc[T::s][v] = (double)raw[T::s][v];
+            if constexpr (UPD && T::J == 0) tile_update(sh.P, T::I, T::J, lr, lj, acc[T::s]);
         }
     });
-    // tile column 0 for panel 0
-    each_slot<W>([&](auto t) {
-        using T = decltype(t);
-        if constexpr (T::ok && T::J == 0) {
+    for (int J = 0; J < DN; ++J) {
+        // ---- phase F
+        const double (*op)[4][64] = sh.op;   // panel J - 1
+        auto apply = [&](auto t) {
+            using T = decltype(t);
+            double a[4], b[4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sh.pRaw[T::I * 16 + lr + 4 * v][lj] = accA[T::s][v];
-        }
-    });
-    __syncthreads();
-    for (int it = 0; it <= 16; ++it) {
-        // ---- phase U
-        if (it >= 1) {
-            // panel p = it - 1: A -= L_p L_p^T on live tiles outside tile
-            // column it >> 1 (updated in phase A of iteration p)
-            const int p = it - 1, skipJ = it >> 1, lim = 8 * p + 8;
-            const double (*P)[DP] = sh.pL[p % PLBUF];
-            double op[8][2];
-#pragma unroll
-            for (int r = 0; r < 8; ++r) load_op(P, r, lr, lj, op[r]);
-            each_slot<W>([&](auto t) {
-                using T = decltype(t);
-                if constexpr (T::ok) {
-                    if (T::J != skipJ && T::J * 16 + 15 >= lim) {
-#pragma unroll
-                        for (int ks = 0; ks < 2; ++ks)
-                            accA[T::s] = __builtin_amdgcn_mfma_f64_16x16x4f64(-op[T::I][ks], op[T::J][ks], accA[T::s],
-                                                                              0, 0, 0);
-                    }
-                }
-            });
-        }
-        if (it >= 2) {
-            // panel q = it - 2: R -= L_q X_q for rows below the panel and
-            // columns up to its end
-            const int q = it - 2, x0 = 8 * q;
-            const double (*P)[DP] = sh.pL[q % PLBUF];
-            double opM[8][2], opX[8][2];
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                load_op(P, r, lr, lj, opM[r]);
-                load_op(sh.rowXt, r, lr, lj, opX[r]);
+            for (int s = 0; s < 4; ++s) {
+                a[s] = op[T::J][s][lane];
+                b[s] = op[T::I][s][lane];
             }
-            each_slot<W>([&](auto t) {
-                using T = decltype(t);
-                if constexpr (T::ok) {
-                    if (T::I * 16 + 15 >= x0 + 8 && T::J * 16 <= x0 + 7) {
 #pragma unroll
-                        for (int ks = 0; ks < 2; ++ks)
-                            accX[T::s] = __builtin_amdgcn_mfma_f64_16x16x4f64(-opM[T::I][ks], opX[T::J][ks],
-                                                                              accX[T::s], 0, 0, 0);
-                    }
-                }
-            });
-        }
-        if (it >= 1) {
-            // rows x0..x0+7 of R (panel it - 1) for wave 0's substitution
-            const int Jx = (it - 1) >> 1, cx = ((it - 1) & 1) * 8;
+            for (int s = 0; s < 4; ++s)
+                acc[T::s] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[s], b[s], acc[T::s], 0, 0, 0);
+        };
+        // the column that is solved next comes first
+        each_slot<W>([&](auto t) {
+            using T = decltype(t);
+            if constexpr (T::ok && T::J >= 1 && T::I > T::J) {
+                if (T::J == J) apply(t);
+            }
+        });
+        if (UPD) {
             each_slot<W>([&](auto t) {
                 using T = decltype(t);
-                if constexpr (T::ok) {
-                    if (T::I == Jx) {
-                        if (cx == 0) {
-                            sh.rowR[lr][T::J * 16 + lj] = accX[T::s][0];
-                            sh.rowR[lr + 4][T::J * 16 + lj] = accX[T::s][1];
-                        } else {
-                            sh.rowR[lr][T::J * 16 + lj] = accX[T::s][2];
-                            sh.rowR[lr + 4][T::J * 16 + lj] = accX[T::s][3];
-                        }
-                    }
+                if constexpr (T::ok && T::J >= 1) {
+                    if (T::J == J + 1) tile_update(sh.P, T::I, T::J, lr, lj, acc[T::s]);
                 }
             });
         }
+        each_slot<W>([&](auto t) {
+            using T = decltype(t);
+            if constexpr (T::ok && T::J >= 2) {
+                if (J >= 1 && T::J > J) apply(t);
+            }
+            if constexpr (T::ok && T::J >= 1 && T::I == T::J) {
+                if (T::J == J + 1) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sh.dg[v][lane] = acc[T::s][v];
+                }
+            }
+        });
+        // panel J - 1 (solved, in the accumulators) to memory, its mirror zeroed
+        each_slot<W>([&](auto t) {
+            using T = decltype(t);
+            if constexpr (T::ok && T::I > T::J) {
+                if (T::J == J - 1) {
+                    double* o = packed + packed_at(T::I, T::J) * PACKED;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int i = T::I * DT + lj, j = T::J * DT + lr + 4 * v;
+                        if (i < nb && j < nb) A[(int64_t)i * ld + j] = (float)acc[T::s][v];
+                        const int mi = T::J * DT + lr + 4 * v, mj = T::I * DT + lj;
+                        if (mi < nb && mj < nb) A[(int64_t)mi * ld + mj] = 0.0f;
+                        // column lr + 4 v: 4 (l/16) + 2 h + e with l/16 = v; row lj = perm16(l%16)
+                        o[((lr >> 1) * 64 + 16 * v + perm16(lj)) * 2 + (lr & 1)] = acc[T::s][v];
+                    }
+                }
+            }
+        });
         lds_barrier();
-        // ---- phase A: panel it's update of the tile column holding panel it + 1, published
-        if (it <= 14) {
-            const int Jn = (it + 1) >> 1;
-            const double (*P)[DP] = sh.pL[it % PLBUF];
-            double opn[2];
-            load_op(P, Jn, lr, lj, opn);
-            each_slot<W>([&](auto t) {
-                using T = decltype(t);
-                if constexpr (T::ok) {
-                    if (T::J == Jn) {
-                        double opi[2];
-                        load_op(P, T::I, lr, lj, opi);
+        // ---- phase S
+        each_slot<W>([&](auto t) {
+            using T = decltype(t);
+            if constexpr (T::ok && T::I > T::J) {
+                if (T::J == J) {
+                    double a[4];
 #pragma unroll
-                        for (int ks = 0; ks < 2; ++ks)
-                            accA[T::s] = __builtin_amdgcn_mfma_f64_16x16x4f64(-opi[ks], opn[ks], accA[T::s], 0, 0, 0);
+                    for (int s = 0; s < 4; ++s) a[s] = sh.inv[lj][lr + 4 * s];
+                    ddoublex4 x = ddoublex4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) sh.pRaw[T::I * 16 + lr + 4 * v][lj] = accA[T::s][v];
-                    }
+                    for (int s = 0; s < 4; ++s) x = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], acc[T::s][s], x, 0, 0, 0);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sh.op[T::I][v][lane] = x[v];
+                    acc[T::s] = x;
                 }
-            });
-        }
-        // columns 64..127 of the rows of X of panel it - 1 (wave 0 does 0..63)
-        if (W == 1 && it >= 1) x_rows(sh, it - 1, 64 + lane, nb, D64);
+            }
+        });
         lds_barrier();
     }
 }
 
-// The diagonal block of matrix b, by a work-group of DIAG_WAVES waves.
+// Wave 0: the diagonal tiles.
+template <bool UPD>
+__device__ __forceinline__ void diag_factor_wave(DiagShared& sh, float* A, int64_t ld, int nb, double* packed,
+                                                 int lane, int& bad) {
+    const int lr = lane >> 4, lj = lane & 15;
+    ddoublex4 acc, Lt, X;
+    float raw[4];
+    load_tile(A, ld, nb, 0, 0, lr, lj, raw);
+    if (UPD) __syncthreads();   // sh.P
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] = (double)raw[v];
+    if (UPD) tile_update(sh.P, 0, 0, lr, lj, acc);
+    for (int J = 0; J < DN; ++J) {
+        if (J > 0) {
+            const double (*op)[64] = sh.op[J];
+            double a[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) a[s] = op[s][lane];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[s], a[s], acc, 0, 0, 0);
+        }
+        factor_tile(acc, Lt, X, lane, J * DT, bad);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sh.inv[lr + 4 * v][lj] = X[v];
+        lds_barrier();
+        if (J + 1 < DN) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[v] = sh.dg[v][lane];
+        }
+        ddoublex2* o = reinterpret_cast<ddoublex2*>(packed + packed_at(J, J) * PACKED) + lane;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const double* q = &sh.inv[perm16(lj)][4 * lr + 2 * h];
+            o[h * 64] = ddoublex2{q[0], q[1]};
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = J * DT + lj, j = J * DT + lr + 4 * v;
+            if (i < nb && j < nb) A[(int64_t)i * ld + j] = (float)Lt[v];
+        }
+        lds_barrier();
+    }
+}
+
+// The diagonal block of matrix b, by a work-group of DIAG_WAVES waves; UPD:
+// updated first with the 128 columns of the panel before it (VEC: its rows
+// are 16-byte aligned).
+template <bool UPD, bool VEC = false>
 __device__ __forceinline__ void diag_block(DiagShared& sh, int b, float* H, int64_t ld, int64_t stride, int64_t k0,
                                            int nb, double* dinv64, int64_t dstride, int* info) {
     float* A = H + (int64_t)b * stride + k0 * ld + k0;
-    double* D64 = dinv64 + (int64_t)b * dstride;
+    double* packed = dinv64 + (int64_t)b * dstride;
     const int lane = threadIdx.x & 63;
-    // uniform in the wave; every wave runs 1 + 2 * 17 barriers
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // the spare row of pRaw starts at 0; the first barrier orders this
-    if (threadIdx.x < RP) sh.pRaw[NB][threadIdx.x] = 0.0;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform
     int bad = 0;
-    switch (wave) {
-        case 0: __syncthreads(); diag_factor_wave(sh, nb, D64, lane, bad); break;
-        case 1: diag_tile_wave<1>(sh, A, ld, nb, D64, lane); break;
-        case 2: diag_tile_wave<2>(sh, A, ld, nb, D64, lane); break;
-        case 3: diag_tile_wave<3>(sh, A, ld, nb, D64, lane); break;
-        case 4: diag_tile_wave<4>(sh, A, ld, nb, D64, lane); break;
-        case 5: diag_tile_wave<5>(sh, A, ld, nb, D64, lane); break;
-        case 6: diag_tile_wave<6>(sh, A, ld, nb, D64, lane); break;
-        default: diag_tile_wave<7>(sh, A, ld, nb, D64, lane); break;
+    if (UPD) {
+        // rows of the panel before the block (columns k0 - NB ..), rows past it as zeros
+        const float* Pg = A - NB;
+        const int r = threadIdx.x >> 5, c = (threadIdx.x & 31) * 4;
+        float v[NB / 16][4];
+#pragma unroll
+        for (int u = 0; u < NB / 16; ++u) {
+            const bool in = r + 16 * u < nb;
+            const float* q = Pg + (int64_t)(in ? r + 16 * u : 0) * ld + c;
+            if (VEC) {
+                const float4 f = *reinterpret_cast<const float4*>(q);
+                v[u][0] = f.x; v[u][1] = f.y; v[u][2] = f.z; v[u][3] = f.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[u][e] = q[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[u][e] = in ? v[u][e] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < NB / 16; ++u)
+            *reinterpret_cast<float4*>(&sh.P[(r + 16 * u) * UP + c]) = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
     }
-    __syncthreads();
-    // write L, row-coalesced: Lfin holds every element on and below the
-    // diagonal (panel p writes rows 8 p .. 127 of its columns); the upper
-    // triangle is 0.  Eight LDS reads in flight per batch of stores.
-    constexpr int PER_THREAD = NB * NB / (DIAG_WAVES * 64);
-#pragma unroll 8
-    for (int u = 0; u < PER_THREAD; ++u) {
-        const int idx = (int)threadIdx.x + u * DIAG_WAVES * 64, i = idx >> 7, j = idx & (NB - 1);
-        const float v = j <= i ? sh.Lfin[i][j] : 0.0f;
-        if (i < nb && j < nb) A[(int64_t)i * ld + j] = v;
+    switch (wave) {
+        case 0: diag_factor_wave<UPD>(sh, A, ld, nb, packed, lane, bad); break;
+        case 1: diag_tile_wave<1, UPD>(sh, A, ld, nb, packed, lane); break;
+        case 2: diag_tile_wave<2, UPD>(sh, A, ld, nb, packed, lane); break;
+        case 3: diag_tile_wave<3, UPD>(sh, A, ld, nb, packed, lane); break;
+        case 5: diag_tile_wave<4, UPD>(sh, A, ld, nb, packed, lane); break;
+        case 6: diag_tile_wave<5, UPD>(sh, A, ld, nb, packed, lane); break;
+        case 7: diag_tile_wave<6, UPD>(sh, A, ld, nb, packed, lane); break;
+        default:
+            if (UPD) __syncthreads();   // then gone: a barrier waits only for the waves still running
+            return;
     }
     if (threadIdx.x == 0 && bad && info[b] == 0) info[b] = (int)k0 + bad;
 }
@@ -474,112 +485,207 @@ __global__ __launch_bounds__(DIAG_WAVES * 64) void potrf_diag_kernel(float* H, i
                                                                     int nb, double* dinv64, int64_t dstride,
                                                                     int* info) {
     __shared__ __attribute__((aligned(16))) DiagShared sh;
-    diag_block(sh, blockIdx.x, H, ld, stride, k0, nb, dinv64, dstride, info);
+    diag_block<false>(sh, blockIdx.x, H, ld, stride, k0, nb, dinv64, dstride, info);
 }
 
-// The diagonal block of matrix blockIdx.z (work-group 0) beside the
-// previous block's update of the rest of its super-block: work-group
-// t >= 1 runs tile t - 1 (REST_T x REST_T) of the GEMM g (batch entry
-// blockIdx.z) on its first four waves, in the LDS the diagonal block uses;
-// the other waves end at once (a barrier waits only for the waves still
-// running).  The two touch disjoint columns.  One launch instead of two,
-// and the update runs while the diagonal block's serial chain does.  The
-// launch holds one work-group per CU (the diagonal block's LDS), where
-// 128-tiles (a quarter as many as 64-tiles) finish the update sooner.
+// The diagonal block of matrix blockIdx.z (work-group 0), which it updates
+// with the previous block's panel first, beside that panel's update of the
+// rest of the super-block: work-group t >= 1 runs tile t (REST_T x REST_T) of
+// the GEMM g (batch entry blockIdx.z; tile 0 is the diagonal block) on its
+// first four waves, in the LDS the diagonal block uses; the other waves end
+// at once (a barrier waits only for the waves still running).  One launch
+// instead of two, and the update runs while the diagonal block's serial chain
+// does.
 constexpr int REST_T = 128;
 static_assert(2 * gk::Geo<REST_T>::TILE_F * sizeof(float) <= sizeof(DiagShared), "GEMM tile staging fits");
+template <bool VEC>
 __global__ __launch_bounds__(DIAG_WAVES * 64) void potrf_diag_rest_kernel(float* H, int64_t ld, int64_t stride,
                                                                          int64_t k0, int nb, double* dinv64,
                                                                          int64_t dstride, int* info, GemmArgs g) {
     __shared__ __attribute__((aligned(16))) DiagShared sh;
     if (blockIdx.x == 0) {
-        diag_block(sh, blockIdx.z, H, ld, stride, k0, nb, dinv64, dstride, info);
+        diag_block<true, VEC>(sh, blockIdx.z, H, ld, stride, k0, nb, dinv64, dstride, info);
         return;
     }
     if (threadIdx.x >= 256) return;
-    const gk::TileRange tr = gk::tile_of<REST_T>(g, blockIdx.x - 1);
+    const gk::TileRange tr = gk::tile_of<REST_T>(g, blockIdx.x);
     if (tr.skip) return;
-    gk::gemm_tile<0, 1, true, REST_T, gk::CHUNK_SUM>(g, tr, blockIdx.z, reinterpret_cast<float*>(&sh));
+    // whole tiles of aligned rows need no checked loads
+    float* lds = reinterpret_cast<float*>(&sh);
+    if (VEC && tr.i0 + REST_T <= g.M && tr.j0 + REST_T <= g.N)
+        gk::gemm_tile<0, 1, false, REST_T, gk::CHUNK_SUM>(g, tr, blockIdx.z, lds);
+    else
+        gk::gemm_tile<0, 1, true, REST_T, gk::CHUNK_SUM>(g, tr, blockIdx.z, lds);
 }
 
-// Panel solve A21 <- A21 * Dinv^T for the m rows below a diagonal block, in
-// place, with fp64 products and accumulation (fp32 in and out).  Multiplying
-// by an explicit inverse is where a blocked fp32 Cholesky loses most
-// accuracy; this step is ~1 % of the factorisation's flops, so it runs on
-// the fp64 matrix cores (v_mfma_f64_16x16x4_f64).
-// Work-group: 64 rows, wave w owning the 16-row strip 16 w .. 16 w + 15 as 8
-// accumulator tiles of 16 columns.  k is staged 32 at a time; a column tile
-// J only takes the k-steps with k <= 16 J + 15 (Dinv is lower triangular).
-constexpr int PR = 64, PK = 32;
-constexpr int PA = PK + 1;   // As pitch (floats)
-constexpr int PD = PK + 2;   // Ds pitch (doubles)
-
-__global__ __launch_bounds__(256) void panel64_kernel(float* A21, int64_t m, int nb, int64_t ld, int64_t stride,
-                                                      const double* dinv64, int64_t dstride) {
-    __shared__ float As[PR * PA];
-    __shared__ double Ds[NB * PD];
-    const int b = blockIdx.y;
-    float* P = A21 + (int64_t)b * stride;
-    const double* D64 = dinv64 + (int64_t)b * dstride;
-    const int64_t r0 = (int64_t)blockIdx.x * PR;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int li = lane & 15, lk = lane >> 4;
-    ddoublex4 acc[8];
-#pragma unroll
-    for (int J = 0; J < 8; ++J) acc[J] = ddoublex4{0.0, 0.0, 0.0, 0.0};
-    // the next chunk's global loads are issued before the current chunk's
-    // MFMAs, so that only the first chunk waits for memory
-    constexpr int NA = PR * PK / 256, ND = NB * PK / 256;
-    float av[NA];
-    double dv[ND];
-    auto load_chunk = [&](int kc) {
-#pragma unroll
-        for (int u = 0; u < NA; ++u) {
-            const int idx = t + u * 256, r = idx / PK, k = idx % PK;
-            const int64_t row = r0 + r;
-            av[u] = (row < m && kc + k < nb) ? P[row * ld + kc + k] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < ND; ++u) {
-            const int idx = t + u * 256, j = idx / PK, k = idx % PK;
-            dv[u] = D64[j * NB + kc + k];
-        }
+// Panel solve A21 <- A21 L^-T for the m rows below a diagonal block, in
+// place, in fp64 (fp32 in and out), by tile columns: with Y = A21^T,
+//   X_J = L_JJ^-1 (Y_J - sum_{K<J} L_JK X_K),
+// 16 rows of A21 at a time as the 16 columns of the MFMA tiles.
+// Bound by the chain of tile columns.  Work-group: `groups` such sets of rows
+// in turn; wave w owns tile columns w and w + 4 of Y and, in registers, the
+// packed tiles that update them.  Step K: its owner forms X_K (a D fragment
+// is a B operand as it stands) and hands it over through LDS; every wave
+// updates its later columns.
+template <int W, bool VEC>
+__device__ __forceinline__ void panel_wave(float* P, int64_t m, int64_t ld, const double* packed, int groups,
+                                           double (&xs)[2][4][64], int lane) {
+    const int lr = lane >> 4, lj = lane & 15;
+    // L tiles of column w (K = 0 .. W) and w + 4 (K = 0 .. W + 4)
+    double l0[W + 1][4], l1[W + 5][4];
+    auto load = [&](double (&o)[4], int J, int K) {
+        const ddoublex2* q = reinterpret_cast<const ddoublex2*>(packed + packed_at(J, K) * PACKED) + lane;
+        const ddoublex2 a = q[0], c = q[64];
+        o[0] = a[0];
+        o[1] = a[1];
+        o[2] = c[0];
+        o[3] = c[1];
     };
-    load_chunk(0);
-    for (int kc = 0; kc < nb; kc += PK) {
-        __syncthreads();
 #pragma unroll
-        for (int u = 0; u < NA; ++u) {
-            const int idx = t + u * 256;
-            As[(idx / PK) * PA + idx % PK] = av[u];
-        }
+    for (int K = 0; K <= W; ++K) load(l0[K], W, K);
 #pragma unroll
-        for (int u = 0; u < ND; ++u) {
-            const int idx = t + u * 256;
-            Ds[(idx / PK) * PD + idx % PK] = dv[u];
-        }
-        __syncthreads();
-        if (kc + PK < nb) load_chunk(kc + PK);
+    for (int K = 0; K <= W + 4; ++K) load(l1[K], W + 4, K);
+    for (int g = 0; g < groups; ++g) {
+        const int64_t row = ((int64_t)blockIdx.x * groups + g) * 16 + lj;
+        const bool in = row < m;
+        float* R = P + (in ? row : 0) * ld + 4 * lr;   // this lane's columns of a tile column: 4 lr .. 4 lr + 3
+        ddoublex4 y[2];
 #pragma unroll
-        for (int ks = 0; ks < PK / 4; ++ks) {
-            const int k = ks * 4 + lk;
-            const double a = (double)As[(wave * 16 + li) * PA + k];
+        for (int o = 0; o < 2; ++o) {
+            float v[4];
+            if (VEC) {
+                const float4 f = *reinterpret_cast<const float4*>(R + (W + 4 * o) * DT);
+                v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+            } else {
 #pragma unroll
-            for (int J = 0; J < 8; ++J) {
-                if (J * 16 + 15 < kc + ks * 4) continue;   // Dinv[j][k] = 0 for k > j
-                const double bb = Ds[(J * 16 + li) * PD + k];
-                acc[J] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bb, acc[J], 0, 0, 0);
+                for (int e = 0; e < 4; ++e) v[e] = R[(W + 4 * o) * DT + e];
             }
-        }
-    }
 #pragma unroll
-    for (int J = 0; J < 8; ++J)
+            for (int e = 0; e < 4; ++e) y[o][e] = in ? (double)v[e] : 0.0;
+        }
+        // X = L_KK^-1 y, to LDS and (fp32) to memory
+        auto solve = [&](int K, const double (&inv)[4], const ddoublex4& yk, ddoublex4& x) {
+            x = ddoublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) x = __builtin_amdgcn_mfma_f64_16x16x4f64(inv[s], yk[s], x, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) xs[K & 1][v][lane] = x[v];
+        };
+        auto store = [&](int K, const ddoublex4& x) {
+            if (!in) return;
+            if (VEC) {
+                *reinterpret_cast<float4*>(R + K * DT) =
+                    make_float4((float)x[0], (float)x[1], (float)x[2], (float)x[3]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) R[K * DT + e] = (float)x[e];
+            }
+        };
+        auto update = [&](const double (&l)[4], const double (&x)[4], ddoublex4& yj) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) yj = __builtin_amdgcn_mfma_f64_16x16x4f64(-l[s], x[s], yj, 0, 0, 0);
+        };
+        auto step = [&](auto kc) {
+            constexpr int K = decltype(kc)::value;
+            ddoublex4 x;
+            if constexpr (K == W) solve(K, l0[W], y[0], x);
+            if constexpr (K == W + 4) solve(K, l1[W + 4], y[1], x);
+            lds_barrier();
+            if constexpr (K == W || K == W + 4) store(K, x);
+            if constexpr (K < W + 4) {
+                double xk[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) xk[v] = xs[K & 1][v][lane];
+                if constexpr (K < W) update(l0[K < W ? K : 0], xk, y[0]);
+                update(l1[K], xk, y[1]);
+            }
+        };
+        static_for<0, DN>(step);
+    }
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(256) void panel_solve_kernel(float* A21, int64_t m, int64_t ld, int64_t stride,
+                                                         const double* dinv64, int64_t dstride, int groups) {
+    __shared__ double xs[2][4][64];
+    float* P = A21 + (int64_t)blockIdx.y * stride;
+    const double* packed = dinv64 + (int64_t)blockIdx.y * dstride;
+    const int lane = threadIdx.x & 63;
+    switch (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {
+        case 0: panel_wave<0, VEC>(P, m, ld, packed, groups, xs, lane); break;
+        case 1: panel_wave<1, VEC>(P, m, ld, packed, groups, xs, lane); break;
+        case 2: panel_wave<2, VEC>(P, m, ld, packed, groups, xs, lane); break;
+        default: panel_wave<3, VEC>(P, m, ld, packed, groups, xs, lane); break;
+    }
+}
+
+// Diagonal blocks of X = L^-1 (128 x 128, fp32, upper part 0) from the packed
+// tiles: block column J on wave J,
+//   X_JJ = L_JJ^-1,  X_IJ = -L_II^-1 sum_{K=J}^{I-1} L_IK X_KJ,
+// each X fragment being the B operand of the products below it.
+template <int J>
+__device__ __forceinline__ void dinv_wave(float* P, int64_t ld, int nb, const double* packed, int lane) {
+    const int lr = lane >> 4, lj = lane & 15;
+    auto store = [&](int I, const ddoublex4& x) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int64_t row = r0 + wave * 16 + lk + 4 * v;
-            const int col = J * 16 + li;
-            if (row < m && col < nb) P[row * ld + col] = (float)acc[J][v];
+            const int i = I * DT + 4 * lr + v, j = J * DT + lj;
+            if (i < nb && j < nb) P[(int64_t)i * ld + j] = (float)x[v];
         }
+    };
+    auto load = [&](int I, int K, double (&o)[4]) {
+        const ddoublex2* q = reinterpret_cast<const ddoublex2*>(packed + packed_at(I, K) * PACKED) + lane;
+        const ddoublex2 a = q[0], c = q[64];
+        o[0] = a[0];
+        o[1] = a[1];
+        o[2] = c[0];
+        o[3] = c[1];
+    };
+    for (int I = 0; I < J; ++I) store(I, ddoublex4{0.0, 0.0, 0.0, 0.0});
+    ddoublex4 x[DN];
+    // L_JJ^-1, row 4 lr + v (D row lr + 4 v in perm16 order), column lj
+    {
+        const double* q = packed + packed_at(J, J) * PACKED;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            x[J][v] = q[((lj >> 1 & 1) * 64 + (lj >> 2) * 16 + (lr + 4 * v)) * 2 + (lj & 1)];
+    }
+    store(J, x[J]);
+#pragma unroll
+    for (int I = J + 1; I < DN; ++I) {
+        ddoublex4 s = ddoublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int K = J; K < I; ++K) {
+            double l[4];
+            load(I, K, l);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s = __builtin_amdgcn_mfma_f64_16x16x4f64(l[u], x[K][u], s, 0, 0, 0);
+        }
+        double l[4];
+        load(I, I, l);
+        x[I] = ddoublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(-l[u], s[u], x[I], 0, 0, 0);
+        store(I, x[I]);
+    }
+}
+
+__global__ __launch_bounds__(512) void dinv_kernel(float* X, int64_t n, int64_t ld, int64_t stride,
+                                                  const double* dinv64, int64_t dstride) {
+    const int64_t k0 = (int64_t)blockIdx.x * NB;
+    const double* packed = dinv64 + (int64_t)blockIdx.y * dstride + (int64_t)blockIdx.x * NB * NB;
+    float* P = X + (int64_t)blockIdx.y * stride + k0 * ld + k0;
+    const int nb = (int)std::min<int64_t>(NB, n - k0), lane = threadIdx.x & 63;
+    switch (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {
+        case 0: dinv_wave<0>(P, ld, nb, packed, lane); break;
+        case 1: dinv_wave<1>(P, ld, nb, packed, lane); break;
+        case 2: dinv_wave<2>(P, ld, nb, packed, lane); break;
+        case 3: dinv_wave<3>(P, ld, nb, packed, lane); break;
+        case 4: dinv_wave<4>(P, ld, nb, packed, lane); break;
+        case 5: dinv_wave<5>(P, ld, nb, packed, lane); break;
+        case 6: dinv_wave<6>(P, ld, nb, packed, lane); break;
+        default: dinv_wave<7>(P, ld, nb, packed, lane); break;
+    }
 }
 
 // Copy the upper triangle onto the lower one (in place), per matrix, in
@@ -632,7 +738,7 @@ double* dinv64_of(float* dinv, int64_t batch, int64_t n) {
 }
 
 // Lower Cholesky in place of `batch` matrices [n, n] (pitch ld, stride sH);
-// dinv64 receives every Dinv_k (batch x nblk x NB x NB, fp64).
+// dinv64 receives every block's packed tiles (batch x nblk x NB x NB doubles).
 //
 // Two-level right-looking: columns are taken in super-blocks of up to
 // SUPER_NB columns.  After each block's panel, only the rest of the
@@ -641,13 +747,12 @@ double* dinv64_of(float* dinv, int64_t batch, int64_t n) {
 // one SYRK per block, with the trailing matrix read and written once per
 // super-block.
 //
-// Look-ahead inside a super-block: block k's update is split into the next
-// block column (before the next diagonal block) and the rest of the
-// super-block, which runs in the next diagonal block's launch
-// (potrf_diag_rest_kernel).  The next block column's update follows that
-// launch, so every element receives the same rank-NB updates in the same
-// order as with one update per block (bit-identical results).
+// Inside a super-block a block costs two launches: its diagonal block, beside
+// the previous block's update of the rest of the super-block (which the
+// diagonal block's work-group applies to the block itself first), and its
+// panel.
 constexpr int64_t SUPER_NB = 1024;
+constexpr int64_t PANEL_GROUPS = 512;   // two work-groups per CU
 
 // Where the split products (split.hpp) are taken instead of gemm_f32's, by
 // the matrix's order alone (a batch's matrices equal each one by itself):
@@ -667,7 +772,8 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
     const int64_t nblk = cdiv(n, NB);
     const int64_t dstride = nblk * NB * NB;
     IC_REQUIRE(batch <= 65535, "potrf: batch too large");
-    bool rest_pending = false;   // `rest`: the previous block's update of the rest of its super-block
+    const bool aligned = (uintptr_t)H % 16 == 0 && ld % 4 == 0 && sH % 4 == 0;
+    bool rest_pending = false;   // `rest`: the previous block's update of its super-block, diagonal block included
     GemmArgs rest{};
     int64_t rest_tiles = 0;
     for (int64_t s0 = 0; s0 < n; s0 += SUPER_NB) {
@@ -680,12 +786,16 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
                 double fl = batch * (2.0 / 3.0) * nb * nb * nb, by = batch * 3.0 * 4 * nb * nb;
                 if (rest_pending) fl += rest.algo_flops, by += 4.0 * batch * (2.0 * rest.M * rest.K + 2.0 * rest.M * rest.N);
                 ProfScope prof_scope(st, PT_DIAG, fl, by);
-                if (rest_pending)
-                    hipLaunchKernelGGL(potrf_diag_rest_kernel, dim3((unsigned)(1 + rest_tiles), 1, (unsigned)batch),
-                                       dim3(DIAG_WAVES * 64), 0, st, H, ld, sH, k0, nb, Dk64, dstride, info, rest);
+                const dim3 gd((unsigned)rest_tiles, 1, (unsigned)batch), wg(DIAG_WAVES * 64);
+                if (rest_pending && aligned)
+                    hipLaunchKernelGGL((potrf_diag_rest_kernel<true>), gd, wg, 0, st, H, ld, sH, k0, nb, Dk64, dstride,
+                                       info, rest);
+                else if (rest_pending)
+                    hipLaunchKernelGGL((potrf_diag_rest_kernel<false>), gd, wg, 0, st, H, ld, sH, k0, nb, Dk64, dstride,
+                                       info, rest);
                 else
-                    hipLaunchKernelGGL(potrf_diag_kernel, dim3((unsigned)batch), dim3(DIAG_WAVES * 64), 0, st, H, ld,
-                                       sH, k0, nb, Dk64, dstride, info);
+                    hipLaunchKernelGGL(potrf_diag_kernel, dim3((unsigned)batch), wg, 0, st, H, ld, sH, k0, nb, Dk64,
+                                       dstride, info);
                 IC_CHECK_LAUNCH();
                 rest_pending = false;
             }
@@ -694,35 +804,31 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
             if (m <= 0) break;
             float* A21 = H + k1 * ld + k0;
             {
-                // panel: A21 <- A21 * Dinv^T (fp64 accumulation, in place)
+                // panel: A21 <- A21 L_kk^-T (in place); at most PANEL_GROUPS work-groups, which then take
+                // several sets of rows each
                 ProfScope prof_scope(st, PT_PANEL, (double)batch * m * nb * (nb + 1), (double)batch * m * nb * 8.0);
-                hipLaunchKernelGGL(panel64_kernel, dim3((unsigned)cdiv(m, PR), (unsigned)batch), dim3(256), 0, st,
-                                   A21, m, nb, ld, sH, Dk64, dstride);
+                const int64_t sets = cdiv(m, 16);
+                const int groups = (int)cdiv(sets, PANEL_GROUPS);
+                const dim3 gd((unsigned)cdiv(sets, groups), (unsigned)batch);
+                if (aligned)
+                    hipLaunchKernelGGL((panel_solve_kernel<true>), gd, dim3(256), 0, st, A21, m, ld, sH, Dk64, dstride,
+                                       groups);
+                else
+                    hipLaunchKernelGGL((panel_solve_kernel<false>), gd, dim3(256), 0, st, A21, m, ld, sH, Dk64, dstride,
+                                       groups);
                 IC_CHECK_LAUNCH();
             }
-            // rest of the super-block: A[k1:, k1:s1] -= A21 A21[:s1-k1]^T (lower in its top square), the
-            // next block column now, the others in the next diagonal block's launch
+            // rest of the super-block: A[k1:, k1:s1] -= A21 A21[:s1-k1]^T (lower in its top square), in the next
+            // diagonal block's launch.  One chunk (K = nb <= kc): C - P in the sum form, as gemm_f32 runs it
             const int64_t w = s1 - k1;
             if (w > 0) {
-                const int64_t la = std::min<int64_t>(NB, w);
-                GemmArgs g{m, la, nb, -1.0f, 1.0f, A21, ld, sH, A21, ld, sH, H + k1 * ld + k1, ld, sH, 0, 1,
-                           CMASK_LOWER, KR_FULL, batch, PT_GEMM_CHOL,
-                           (double)batch * 2.0 * (dtri((double)la) + (double)(m - la) * la) * nb};
-                g.chunk_sub = 1;   // a sequence of rank-128 updates, like LAPACK's blocked potrf
-                int rc = gemm_f32(g, st);
-                if (rc) return rc;
-                if (w > la) {
-                    // one chunk (K = nb <= kc): C - P in the sum form, as gemm_f32 runs it
-                    const float* A2 = A21 + la * ld;
-                    rest = GemmArgs{m - la, w - la, nb, -1.0f, 1.0f, A2, ld, sH, A2, ld, sH,
-                                    H + (k1 + la) * ld + k1 + la, ld, sH, 0, 1, CMASK_LOWER, KR_FULL, batch,
-                                    PT_GEMM_CHOL,
-                                    (double)batch * 2.0 * (dtri((double)(w - la)) + (double)(m - w) * (w - la)) * nb};
-                    bool tri;
-                    rest_tiles = gk::tile_count<REST_T>(rest, tri);
-                    IC_REQUIRE(rest_tiles < (1LL << 30), "potrf: problem too large");
-                    rest_pending = true;
-                }
+                rest = GemmArgs{m, w, nb, -1.0f, 1.0f, A21, ld, sH, A21, ld, sH, H + k1 * ld + k1, ld, sH, 0, 1,
+                                CMASK_LOWER, KR_FULL, batch, PT_GEMM_CHOL,
+                                (double)batch * 2.0 * (dtri((double)w) + (double)(m - w) * w) * nb};
+                bool tri;
+                rest_tiles = gk::tile_count<REST_T>(rest, tri);
+                IC_REQUIRE(rest_tiles < (1LL << 30), "potrf: problem too large");
+                rest_pending = true;
             }
         }
         // beyond the super-block: A[s1:, s1:] -= L[s1:, s0:s1] L[s1:, s0:s1]^T (lower)
@@ -768,30 +874,6 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
 // upper block of the merged square.  All pairs of one level that have the same shape run as one
 // batched GEMM, so the whole inverse takes ~2 log2(n/128) launches of
 // large-K GEMMs instead of 2 n/128 rank-128 updates.
-__global__ void put_diag_all_kernel(float* X, int64_t n, int64_t ld, int64_t stride, const double* dinv64,
-                                    int64_t dstride) {
-    const int64_t k0 = (int64_t)blockIdx.x * NB;
-    const int b = blockIdx.y;
-    const double* D = dinv64 + (int64_t)b * dstride + (int64_t)blockIdx.x * NB * NB;
-    float* P = X + (int64_t)b * stride + k0 * ld + k0;
-    const int nb = (int)std::min<int64_t>(NB, n - k0);
-    if (nb == NB && ld % 4 == 0 && (reinterpret_cast<uintptr_t>(P) & 15) == 0) {
-        // whole block, 16-byte rows: 32 float4 per row, each from 4 doubles
-        for (int idx = threadIdx.x; idx < NB * NB / 4; idx += blockDim.x) {
-            const int i = idx >> 5, j4 = (idx & 31) * 4;
-            const double2 a = *reinterpret_cast<const double2*>(&D[i * NB + j4]);
-            const double2 c = *reinterpret_cast<const double2*>(&D[i * NB + j4 + 2]);
-            *reinterpret_cast<float4*>(&P[(int64_t)i * ld + j4]) =
-                make_float4((float)a.x, (float)a.y, (float)c.x, (float)c.y);
-        }
-        return;
-    }
-    for (int idx = threadIdx.x; idx < nb * nb; idx += blockDim.x) {
-        const int i = idx / nb, j = idx - i * nb;
-        P[(int64_t)i * ld + j] = (float)D[i * NB + j];
-    }
-}
-
 static int merge_pairs(const float* L, float* X, int64_t ld, int64_t r0, int64_t n1, int64_t n2, int64_t count,
                        int64_t pstride, int64_t batch, int64_t sH, hipStream_t st) {
     // per (pair, matrix): strides differ only when both are > 1; then loop over matrices
@@ -885,8 +967,8 @@ int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_
           hipStream_t st, const SplitWork* w) {
     const int64_t nblk = cdiv(n, NB);
     const int64_t dstride = nblk * NB * NB;
-    hipLaunchKernelGGL(put_diag_all_kernel, dim3((unsigned)nblk, (unsigned)batch), dim3(256), 0, st, X, n, ld, sH,
-                       dinv64, dstride);
+    hipLaunchKernelGGL(dinv_kernel, dim3((unsigned)nblk, (unsigned)batch), dim3(512), 0, st, X, n, ld, sH, dinv64,
+                       dstride);
     IC_CHECK_LAUNCH();
     // segments of rows [start, start + len); merged pairwise per level
     std::vector<int64_t> seg;
