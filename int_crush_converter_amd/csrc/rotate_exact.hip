@@ -96,6 +96,7 @@ __device__ __forceinline__ void flush_zeroed(unsigned cnt, unsigned long long* n
 
 constexpr int XR_ROWS = 64;            // rows per tile (4 row tiles of 16 per MFMA)
 constexpr int XR_SLICE = 256;          // output columns per work-group: 4 waves x 4 tiles x 16
+constexpr int XN_ROWS = 16;            // rows (columns) per work-group of the narrow kernels
 constexpr int XR_LD = XR_SLICE + 4;    // LDS pitch: lanes 4 banks apart, 16-byte reads conflict-free
 
 // Work-group y takes output columns [s0, s0 + 256) of every 64-row tile
@@ -276,6 +277,80 @@ __global__ __launch_bounds__(256, 2) void rot_rows_exact_kernel(const void* __re
         ch = nch;
     }
     if (count) flush_zeroed(cnt, nz);
+}
+
+// The row kernel for launches that leave most of the chip idle (R = 64, 256):
+// work-group = 16 rows x one 256-column slice, wave w its columns 64 w .. + 63
+// in ONE accumulator: the four blocks of an MFMA are four column tiles (not
+// four row tiles), A = X is the same in all of them.  A quarter of the wide
+// kernel's work per wave on four times the work-groups, the same chain per
+// output.  Block b = lane / 16 is the column tile, so the sign's second part
+// (see the row kernel) is per lane and flips A with the uniform third.
+// In place is safe: a work-group reads its whole rows of the slice first.
+template <int R, int DT>
+__global__ __launch_bounds__(256) void rot_rows_narrow_kernel(const void* src, int64_t rows, int64_t cols,
+                                                             int64_t ld_src, float* dst, int64_t cols_pad,
+                                                             int64_t ld_dst, int64_t n_tri, uint32_t mag_bits,
+                                                             float zero_above, unsigned long long* nz, int vec) {
+    static_assert(R == 64 || R == 256, "four column tiles of one group per wave");
+    constexpr bool REG = (R & 0x55555555) == R;
+    __shared__ __align__(16) float xs[XN_ROWS * XR_LD];
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lb = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t s0 = (int64_t)blockIdx.y * XR_SLICE, r0 = (int64_t)blockIdx.x * XN_ROWS;
+    if (n_tri > 0 && s0 / R > r0 / R) return;   // only blocks on and below the diagonal are needed
+    float v[4][4];
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        const int u = it * 256 + tid, rr = u >> 6, cq = (u & 63) * 4;
+        const int64_t r = r0 + rr, c = s0 + cq;
+        if (r < rows) load4<DT>(src, r * ld_src + c, c, cols, (vec & 1) != 0, v[it]);
+        else v[it][0] = v[it][1] = v[it][2] = v[it][3] = 0.0f;
+    }
+    float bp[16];   // m (-1)^s(q, lane & 15)
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+        bp[q] = __uint_as_float(mag_bits | (hd_sign<REG>((uint32_t)q, (uint32_t)li) << 31));
+    uint32_t sb[4];   // s(kh & 3, b) as a sign bit
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sb[k] = hd_sign<REG>((uint32_t)k, (uint32_t)lb) << 31;
+    unsigned cnt = 0;
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        if (zero_above > 0.0f) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool out = fabsf(v[it][i]) > zero_above;
+                cnt += out ? 1u : 0u;
+                v[it][i] = out ? 0.0f : v[it][i];
+            }
+        }
+        const int u = it * 256 + tid, rr = u >> 6, cq = (u & 63) * 4;
+        *reinterpret_cast<float4*>(&xs[rr * XR_LD + cq]) = make_float4(v[it][0], v[it][1], v[it][2], v[it][3]);
+    }
+    __syncthreads();
+    const float* xrow = &xs[li * XR_LD + (64 * w) / R * R];
+    const uint32_t uhi = R == 256 ? (uint32_t)w : 0u;
+    f32x16 acc = f32x16{};
+    float4 an = *reinterpret_cast<const float4*>(xrow);
+    auto step = [&](auto TT) {
+        constexpr int t = decltype(TT)::value, kh = t / 4, q4 = t % 4;
+        float4 a = an;
+        if constexpr (t + 1 < R / 4) an = *reinterpret_cast<const float4*>(xrow + 4 * (t + 1));
+        const uint32_t gs = sb[kh & 3] ^ (R == 256 ? hd_sign<REG>((uint32_t)kh >> 2, uhi) << 31 : 0u);
+        float x[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = __uint_as_float(__float_as_uint(x[i]) ^ gs);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc = mfma_k1(x[i], bp[4 * q4 + i], acc);
+    };
+    static_for<0, R / 4>(step);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int64_t r = r0 + 4 * lb + (e & 3), c = s0 + 64 * w + 16 * (e >> 2) + li;
+        if (r < rows && c < cols_pad) dst[r * ld_dst + c] = acc[e];
+    }
+    if (zero_above > 0.0f) flush_zeroed(cnt, nz);
 }
 
 // Rows out of place, one wave per output slice (R = 64, 128, 256; rows whose
@@ -591,6 +666,64 @@ __global__ __launch_bounds__(256, 2) void rot_cols_exact_kernel(const float* __r
     }
 }
 
+// The column kernel's counterpart of rot_rows_narrow_kernel: work-group = 256
+// rows x 16 columns, wave w rows 64 w .. + 63 in one accumulator: the blocks
+// are four row tiles p (A = the Hadamard entries), B = the same 16 columns in
+// all of them, flipped per lane by the sign's second part.
+template <int R>
+__global__ __launch_bounds__(256) void rot_cols_narrow_kernel(const float* src, float* dst, int64_t n, int64_t ld,
+                                                             int64_t bstride, int tri, uint32_t mag_bits, int vec) {
+    static_assert(R == 64 || R == 256, "four row tiles of one group per wave");
+    constexpr bool REG = (R & 0x55555555) == R;
+    __shared__ __align__(16) float hs[XC_ROWS * XN_ROWS];
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lb = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t r0 = (int64_t)blockIdx.y * XC_ROWS, l0 = (int64_t)blockIdx.x * XN_ROWS;
+    if (tri && l0 / R > std::min<int64_t>(r0 + XC_ROWS - 1, n - 1) / R) return;
+    const float* S = src + (int64_t)blockIdx.z * bstride;
+    float* D = dst + (int64_t)blockIdx.z * bstride;
+    float v[4][4];
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        const int u = it * 256 + tid, rr = u >> 2, cq = (u & 3) * 4;
+        const int64_t r = r0 + rr, c = l0 + cq;
+        if (r < n) load4<IC_DTYPE_F32>(S, r * ld + c, c, n, (vec & 1) != 0, v[it]);
+        else v[it][0] = v[it][1] = v[it][2] = v[it][3] = 0.0f;
+    }
+    float ap[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+        ap[q] = __uint_as_float(mag_bits | (hd_sign<REG>((uint32_t)q, (uint32_t)li) << 31));
+    uint32_t sb[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sb[k] = hd_sign<REG>((uint32_t)k, (uint32_t)lb) << 31;
+#pragma unroll
+    for (int it = 0; it < 4; ++it)
+        *reinterpret_cast<float4*>(&hs[(it * 256 + tid) * 4]) = make_float4(v[it][0], v[it][1], v[it][2], v[it][3]);
+    __syncthreads();
+    const float* hcol = &hs[(64 * w) / R * R * XN_ROWS + li];
+    const uint32_t uhi = R == 256 ? (uint32_t)w : 0u;
+    f32x16 acc = f32x16{};
+    constexpr int PF = 8;   // B values read ahead
+    float bn[PF];
+#pragma unroll
+    for (int t = 0; t < PF; ++t) bn[t] = hcol[t * XN_ROWS];
+    auto step = [&](auto TT) {
+        constexpr int t = decltype(TT)::value, kh = t / 16, q = t % 16;
+        float b = bn[t % PF];
+        if constexpr (t + PF < R) bn[t % PF] = hcol[(t + PF) * XN_ROWS];
+        const uint32_t gs = sb[kh & 3] ^ (R == 256 ? hd_sign<REG>((uint32_t)kh >> 2, uhi) << 31 : 0u);
+        b = __uint_as_float(__float_as_uint(b) ^ gs);
+        acc = mfma_k1(ap[q], b, acc);
+    };
+    static_for<0, R>(step);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int64_t r = r0 + 64 * w + 16 * (e >> 2) + 4 * lb + (e & 3), c = l0 + li;
+        if (r < n && c < n) D[r * ld + c] = acc[e];
+    }
+}
+
 // ------------------------------------------------------------------ small R (2, 4, 8): VALU fma chains
 
 // One thread per (row, group): reads the group's R inputs, writes its R
@@ -664,6 +797,15 @@ static float hd_mag(int rot) {
 // work-groups a launch aims at (four per CU: two resident, two queued)
 constexpr int64_t XR_WGS = 1024;
 
+// Launches of at most this many wide work-groups (64 rows x 256 columns; half
+// a chip's) take the narrow kernels: a wide one's chain of 4 x R MFMAs per wave
+// is then the launch (R = 256: 19-25 us at any size up to it), where a narrow
+// one's is a quarter.  Measured: weights [64, 256] 19.0 -> 9.2 us, [256, 1024]
+// 21.3 -> 10.7; a 1024 x 1024 Hessian's columns 25.0 -> 13.0, rows 23.0 ->
+// 10.7.  Beyond half a chip the narrow work-groups share CUs and save nothing.
+constexpr int64_t XN_MAX = 128;
+static bool narrow(int64_t wide_wgs, int rot) { return wide_wgs <= XN_MAX && (rot == 64 || rot == 256); }
+
 static int small_grid(int64_t work) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(cdiv(work, 256), 256 * 32));
 }
@@ -710,6 +852,20 @@ static int rows_exact(const void* src, int dt, int64_t rows, int64_t cols, int64
                            else if (dt == IC_DTYPE_F32) ICQ_XR(RR, IC_DTYPE_F32, false); \
                            else if (dt == IC_DTYPE_BF16) ICQ_XR(RR, IC_DTYPE_BF16, false); \
                            else ICQ_XR(RR, IC_DTYPE_F16, false); } while (0)
+    if (narrow(ntile * slices, rot)) {
+        const dim3 ng((unsigned)cdiv(rows, XN_ROWS), (unsigned)slices);
+#define ICQ_XN(RR, D) hipLaunchKernelGGL((rot_rows_narrow_kernel<RR, D>), ng, dim3(256), 0, st, src, rows, cols, \
+                                         ld_src, dst, cols_pad, ld_dst, n_tri, mb, zero_above, nz, vec)
+#define ICQ_XN_DT(RR) do { if (dt == IC_DTYPE_F32) ICQ_XN(RR, IC_DTYPE_F32); \
+                           else if (dt == IC_DTYPE_BF16) ICQ_XN(RR, IC_DTYPE_BF16); \
+                           else ICQ_XN(RR, IC_DTYPE_F16); } while (0)
+        if (rot == 64) ICQ_XN_DT(64);
+        else ICQ_XN_DT(256);
+#undef ICQ_XN_DT
+#undef ICQ_XN
+        IC_CHECK_LAUNCH();
+        return IC_OK;
+    }
     // rot_rows_wave_kernel's domain: out of place, whole groups, vector loads
     const bool wave = !tri && src != (const void*)dst && (vec & 1) && cols == cols_pad;
 #define ICQ_XW(RR, D, Z) launch_rows_wave<RR, D, Z>(src, rows, cols, ld_src, dst, cols_pad, ld_dst, mb, zero_above, \
@@ -795,7 +951,15 @@ extern "C" int ic_rotate_hessian_exact(const float* src, float* H, int64_t batch
                                                     n, ld, n * ld, mb, vec); \
                         else hipLaunchKernelGGL((rot_cols_exact_kernel<RR, false>), grid, dim3(256), 0, st, src, H, \
                                                 n, ld, n * ld, mb, vec); } while (0)
-        if (rot == 16) ICQ_XC(16);
+        if (narrow(ntile * nrow * batch, rot)) {
+            const dim3 ng((unsigned)cdiv(n, XN_ROWS), (unsigned)nrow, (unsigned)batch);
+            if (rot == 64)
+                hipLaunchKernelGGL((rot_cols_narrow_kernel<64>), ng, dim3(256), 0, st, src, H, n, ld, n * ld, (int)tri,
+                                   mb, vec);
+            else
+                hipLaunchKernelGGL((rot_cols_narrow_kernel<256>), ng, dim3(256), 0, st, src, H, n, ld, n * ld,
+                                   (int)tri, mb, vec);
+        } else if (rot == 16) ICQ_XC(16);
         else if (rot == 64) ICQ_XC(64);
         else ICQ_XC(256);
 #undef ICQ_XC
