@@ -14,10 +14,22 @@ from .dlr import is_dlr, validate_dlr
 from .log import logger
 
 
-def load_calibration(path: str) -> dict:
-    """Load and validate a calibration file (reference calibration_io.py:9-37)."""
+def load_calibration(path: str, *, mmap: bool = False) -> dict:
+    """Load and validate a calibration file (reference calibration_io.py:9-37).
+    ``mmap``: the tensors are mapped from the file and read as they are used
+    (the file must stay as it is meanwhile); files that cannot be mapped are
+    read whole."""
     try:
-        data = torch.load(path, map_location="cpu", weights_only=True)
+        data = None
+        if mmap:
+            try:
+                data = torch.load(path, map_location="cpu", weights_only=True, mmap=True)
+            except FileNotFoundError:
+                raise
+            except Exception:
+                pass   # not a zip archive, or damaged: the plain load reads it or says what is wrong
+        if data is None:
+            data = torch.load(path, map_location="cpu", weights_only=True)
     except FileNotFoundError:
         raise ValueError(f"Calibration file not found: {path}")
     except Exception as e:
