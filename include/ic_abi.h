@@ -313,8 +313,10 @@ int ic_ls_scales(const int8_t* Q, const float* W, int64_t rows, int64_t cols, fl
  * per row (scale_kind 0: scale[rows]) or per element (scale_kind 1:
  * scale[rows, cols], the reference's scale_2d), H [cols, cols] fp32;
  * Q (int8 [rows, cols]) updated in place.
- * Column blocks of 64 take their cross terms from one fp32-MFMA GEMM plus
- * exact in-block corrections.  workspace: ic_greedy_workspace_bytes().
+ * Column blocks of 64 take their cross terms from one GEMM over all of err
+ * (fp32 MFMA; bf16 MFMA on exactly split operands when rows and cols >= 2048
+ * and cols % 512 == 0, whose planes add 6 (rows + cols) cols bytes to the
+ * workspace, up to 64 GiB) plus exact in-block corrections.  workspace: ic_greedy_workspace_bytes().
  * Replaces converter/greedy.py:487-541 (greedy_local_search_pytorch) and
  * 207-285 (greedy_local_search_triton). */
 int64_t ic_greedy_workspace_bytes(int64_t rows, int64_t cols);

@@ -9,6 +9,7 @@
 // sum_j' d_j' H[j', j] - the same quantity in exact arithmetic as the
 // reference's per-column GEMV (its fp32 rounding differs).
 #include "gemm.hpp"
+#include "split.hpp"
 #include "torchsum.hpp"
 
 namespace icq {
@@ -498,8 +499,11 @@ constexpr int PROXY_PARTS = 1024;
 constexpr int GSPLIT = 4;
 
 // C[r][c] = ((P_0 + P_1) + P_2) + P_3 for the GSPLIT partial products
-// (pitch GSB, stride rows * GSB).
-__global__ void split_sum_kernel(const float* __restrict__ P, int64_t rows, int64_t sw, float* __restrict__ C) {
+// (pitch GSB, stride rows * GSB).  err (or null): P came from split operands,
+// where an infinity gives a NaN; such sums are formed again in fp32 from err's
+// and Hsb's rows (pitch cols), so that a NaN here is one of theirs.
+__global__ void split_sum_kernel(const float* __restrict__ P, int64_t rows, int64_t sw, float* __restrict__ C,
+                                 const float* __restrict__ err, const float* __restrict__ Hsb, int64_t cols) {
     const int64_t total = rows * sw, stride = rows * GSB;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
          i += (int64_t)gridDim.x * blockDim.x) {
@@ -507,26 +511,80 @@ __global__ void split_sum_kernel(const float* __restrict__ P, int64_t rows, int6
         float v = P[o];
 #pragma unroll
         for (int k = 1; k < GSPLIT; ++k) v = v + P[k * stride + o];
+        if (err && !(fabsf(v) <= 3.402823466e38f)) {
+            v = 0.0f;
+            for (int64_t j = 0; j < cols; ++j) v = __builtin_fmaf(err[r * cols + j], Hsb[c * cols + j], v);
+        }
         C[o] = v;
     }
 }
 
+// Large searches form the cross terms from split operands (split.hpp): H's
+// planes once, err's kept up to date super-block by super-block.  The product
+// of a super-block, bounded by the fp32 MFMA rate before, took 148 us at
+// [4096, 4096] and takes 83 on the bf16 pipes, for 10 us of splitting.  The
+// line, five passes (general -> split, us): [4096, 4096] 16900 -> 15209,
+// [2048, 4096] 14026 -> 12851, [4096, 8192] 41900 -> 33934, [2048, 2048] 3662 ->
+// 3511; but [1024, 4096] 11805 -> 11970, [64, 8192] 19108 -> 21390, where H's
+// planes and a few tiles' latency cost more than the product.
+constexpr int64_t GREEDY_SPLIT_COLS = 2048, GREEDY_SPLIT_ROWS = 2048, GREEDY_SPLIT_MAX_BYTES = 64LL << 30;
+struct GreedyPlanes {
+    SplitPlanes E, H;   // err by rows, H by rows
+};
+// Bytes of the planes (0: the general path), and (w) their places from `base` on.
+static int64_t greedy_plane_bytes(int64_t rows, int64_t cols, char* base, GreedyPlanes* w) {
+    if (cols % (GSPLIT * SP_ROWS) || cols < GREEDY_SPLIT_COLS || rows < GREEDY_SPLIT_ROWS) return 0;
+    const int64_t kc = cols / SP_K, e = cdiv(rows, SP_ROWS) * kc * SP_CHUNK, h = cols / SP_ROWS * kc * SP_CHUNK;
+    if ((e + h) * (int64_t)sizeof(uint16_t) > GREEDY_SPLIT_MAX_BYTES) return 0;
+    if (w) {
+        uint16_t* p = reinterpret_cast<uint16_t*>((reinterpret_cast<uintptr_t>(base) + 255) & ~(uintptr_t)255);
+        w->E = SplitPlanes{p, SP_RECT, kc, 0};
+        w->H = SplitPlanes{p + e, SP_RECT, kc, 0};
+    }
+    return (e + h) * (int64_t)sizeof(uint16_t) + 256;
+}
+
 // part: scratch for the split products (GSPLIT * rows * GSB floats), or null.
-// sc / pe: the scales, per row (pe 0) or per element (pe 1).
+// sc / pe: the scales, per row (pe 0) or per element (pe 1).  pl: planes of err
+// and Hc, or null.
 static int greedy_pass(float* err, float* Qf, const float* sc, int pe, const float* Hc, const float* hd, float* C,
-                       float* part, int64_t rows, int64_t cols, float qmin, float qmax, hipStream_t st) {
+                       float* part, int64_t rows, int64_t cols, float qmin, float qmax, const GreedyPlanes* pl,
+                       hipStream_t st) {
     for (int64_t s0 = 0; s0 < cols; s0 += GSB) {
         const int64_t sw = std::min<int64_t>(GSB, cols - s0);
         const int64_t ks = cols / GSPLIT;
         const bool split = part && cols % (GSPLIT * 128) == 0 && cdiv(rows, 128) * cdiv(sw, 128) < 256 &&
                            ks >= 1024;
         int rc;
-        if (split) {
+        if (pl) {
+            SplitGemm g{};
+            g.M = rows;
+            g.N = sw;
+            g.K = ks;
+            g.alpha = 1.0f;
+            g.A.s = pl->E;
+            g.B.s = pl->H;
+            g.B.r0 = s0 / SP_ROWS;
+            g.A.zc = g.B.zc = ks / SP_K;
+            g.C = part;
+            g.ldc = GSB;
+            g.sC = rows * GSB;
+            g.cmask = CMASK_FULL;
+            g.krange = KR_FULL;
+            g.batch = GSPLIT;
+            g.tag = PT_GEMM_GREEDY;
+            g.algo_flops = 2.0 * rows * sw * cols;
+            if ((rc = split_gemm(g, st))) return rc;
+            hipLaunchKernelGGL(split_sum_kernel, dim3(egrid(rows * sw)), dim3(256), 0, st, part, rows, sw, C, err,
+                               Hc + s0 * cols, cols);
+            IC_CHECK_LAUNCH();
+        } else if (split) {
             GemmArgs g{rows, sw, ks, 1.0f, 0.0f, err, cols, ks, Hc + s0 * cols, cols, ks, part, GSB, rows * GSB,
                        0, 1, CMASK_FULL, KR_FULL, GSPLIT, PT_GEMM_GREEDY};
             g.algo_flops = 2.0 * rows * sw * cols;
             if ((rc = gemm_f32(g, st))) return rc;
-            hipLaunchKernelGGL(split_sum_kernel, dim3(egrid(rows * sw)), dim3(256), 0, st, part, rows, sw, C);
+            hipLaunchKernelGGL(split_sum_kernel, dim3(egrid(rows * sw)), dim3(256), 0, st, part, rows, sw, C,
+                               nullptr, nullptr, 0);
             IC_CHECK_LAUNCH();
         } else {
             GemmArgs g{rows, sw, cols, 1.0f, 0.0f, err, cols, 0, Hc + s0 * cols, cols, 0, C, GSB, 0, 0, 1,
@@ -545,6 +603,11 @@ static int greedy_pass(float* err, float* Qf, const float* sc, int pe, const flo
             }
 #undef ICQ_GSB
             IC_CHECK_LAUNCH();
+        }
+        if (pl) {   // the columns that changed
+            int rc2 = split_planes(err, rows, cols, 0, 0, rows, s0, s0 + sw, 0, 0, pl->E, 1, PT_GEMM_GREEDY, st, 1, 0,
+                                   cols);
+            if (rc2) return rc2;
         }
     }
     return IC_OK;
@@ -604,7 +667,8 @@ extern "C" int ic_ls_scales(const int8_t* Q, const float* W, int64_t rows, int64
 }
 
 extern "C" int64_t ic_greedy_workspace_bytes(int64_t rows, int64_t cols) {
-    return (2 * rows * cols + rows * GSB + GSPLIT * rows * GSB) * (int64_t)sizeof(float) + 256;
+    return (2 * rows * cols + rows * GSB + GSPLIT * rows * GSB) * (int64_t)sizeof(float) + 256 +
+           greedy_plane_bytes(rows, cols, nullptr, nullptr);
 }
 
 extern "C" int ic_greedy(const float* W, int8_t* Q, const float* scale, int scale_kind, const float* H, int64_t rows,
@@ -622,8 +686,16 @@ extern "C" int ic_greedy(const float* W, int8_t* Q, const float* scale, int scal
                        cols, err, Qf);
     IC_CHECK_LAUNCH();
     float* part = cross + rows * GSB;
+    GreedyPlanes planes, *pl = nullptr;
+    if (passes > 0 && greedy_plane_bytes(rows, cols, reinterpret_cast<char*>(part + GSPLIT * rows * GSB), &planes)) {
+        pl = &planes;
+        int rc = split_planes(H, cols, cols, 0, 0, cols, 0, cols, 0, 0, pl->H, 1, PT_GEMM_GREEDY, st);
+        if (!rc)
+            rc = split_planes(err, rows, cols, 0, 0, rows, 0, cols, 0, 0, pl->E, 1, PT_GEMM_GREEDY, st, 1, 0, cols);
+        if (rc) return rc;
+    }
     for (int p = 0; p < passes; ++p) {
-        int rc = greedy_pass(err, Qf, scale, scale_kind, H, nullptr, cross, part, rows, cols, qmin, qmax, st);
+        int rc = greedy_pass(err, Qf, scale, scale_kind, H, nullptr, cross, part, rows, cols, qmin, qmax, pl, st);
         if (rc) return rc;
     }
     hipLaunchKernelGGL(to_int8_kernel, dim3(egrid(rows * cols)), dim3(256), 0, st, Qf, rows * cols, qmin, qmax, Q);
@@ -677,7 +749,8 @@ extern "C" int ic_greedy_lowrank(const float* W, int8_t* Q, const float* scale, 
     double prev = 0.0;
     int done = 0;
     for (int p = 0; p < passes; ++p) {
-        int rc = greedy_pass(err, Qf, scale, scale_kind, Hk, hd, cross, split_part, rows, cols, qmin, qmax, st);
+        int rc = greedy_pass(err, Qf, scale, scale_kind, Hk, hd, cross, split_part, rows, cols, qmin, qmax, nullptr,
+                             st);
         if (rc) return rc;
         done = p + 1;
         if (p + 1 == passes) break;   // a stall test after the last pass changes nothing

@@ -273,8 +273,8 @@ __device__ __forceinline__ void store_octet(uint16_t* chunk, int oct, int row, c
 // grid (column blocks, row blocks, squares x batch): the blocks from
 // (rb0, cb0), of `squares` such regions `step` blocks apart along the diagonal.
 template <bool TRANS, bool VEC>
-__global__ __launch_bounds__(256) void split_planes_kernel(const float* A, int64_t n, int64_t ld, int64_t sA,
-                                                          int64_t rb0, int64_t cb0, int lower, int squares,
+__global__ __launch_bounds__(256) void split_planes_kernel(const float* A, int64_t n, int64_t nc, int64_t ld,
+                                                          int64_t sA, int64_t rb0, int64_t cb0, int lower, int squares,
                                                           int64_t step, SplitPlanes out) {
     const int64_t m = blockIdx.z / squares, sq = blockIdx.z - m * squares;
     const int64_t rb = rb0 + blockIdx.y + sq * step, cb = cb0 + blockIdx.x + sq * step;
@@ -295,20 +295,20 @@ __global__ __launch_bounds__(256) void split_planes_kernel(const float* A, int64
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int64_t i = rb * SP_ROWS + oct * 8 + e;
-                x[e] = i < n && j < n ? P[i * ld + j] : 0.0f;
+                x[e] = i < n && j < nc ? P[i * ld + j] : 0.0f;
             }
         } else {
             oct = (idx & 7) + 8 * (idx >> 10);
             row = (idx >> 3) & 127;
             const int64_t i = rb * SP_ROWS + row, j = cb * SP_ROWS + oct * 8;
-            if (VEC && i < n && j + 8 <= n) {
+            if (VEC && i < n && j + 8 <= nc) {
                 const float4 a = *reinterpret_cast<const float4*>(&P[i * ld + j]);
                 const float4 b = *reinterpret_cast<const float4*>(&P[i * ld + j + 4]);
                 x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
                 x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = i < n && j + e < n ? P[i * ld + j + e] : 0.0f;
+                for (int e = 0; e < 8; ++e) x[e] = i < n && j + e < nc ? P[i * ld + j + e] : 0.0f;
             }
         }
         store_octet(o + (oct >> 1) * SP_CHUNK, oct & 1, row, x);
@@ -343,7 +343,7 @@ int split_gemm(const SplitGemm& g, hipStream_t st) {
 
 int split_planes(const float* A, int64_t n, int64_t ld, int64_t sA, int64_t r0, int64_t r1, int64_t c0, int64_t c1,
                  int transpose, int lower, const SplitPlanes& out, int64_t batch, int tag, hipStream_t st,
-                 int64_t squares, int64_t step) {
+                 int64_t squares, int64_t step, int64_t ncols) {
     if (r1 <= r0 || c1 <= c0 || batch <= 0) return IC_OK;
     IC_REQUIRE(r0 % SP_ROWS == 0 && c0 % SP_ROWS == 0, "split_planes: unaligned block");
     const int64_t rbs = cdiv(r1 - r0, SP_ROWS), cbs = cdiv(c1 - c0, SP_ROWS);
@@ -352,9 +352,10 @@ int split_planes(const float* A, int64_t n, int64_t ld, int64_t sA, int64_t r0, 
     ProfScope prof_scope(st, tag, 0.0, 10.0 * batch * squares * (r1 - r0) * (c1 - c0));
     const dim3 gd((unsigned)cbs, (unsigned)rbs, (unsigned)(batch * squares));
     const int64_t rb0 = r0 / SP_ROWS, cb0 = c0 / SP_ROWS;
-#define ICQ_SPLIT(TR, VE)                                                                                        \
-    hipLaunchKernelGGL((split_planes_kernel<TR, VE>), gd, dim3(256), 0, st, A, n, ld, sA, rb0, cb0, lower, \
-                       (int)squares, step / SP_ROWS, out)
+    if (ncols < 0) ncols = n;
+#define ICQ_SPLIT(TR, VE)                                                                                   \
+    hipLaunchKernelGGL((split_planes_kernel<TR, VE>), gd, dim3(256), 0, st, A, n, ncols, ld, sA, rb0, cb0, \
+                       lower, (int)squares, step / SP_ROWS, out)
     if (transpose) ICQ_SPLIT(true, false);
     else if (vec) ICQ_SPLIT(false, true);
     else ICQ_SPLIT(false, false);

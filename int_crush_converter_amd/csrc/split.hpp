@@ -63,14 +63,14 @@ struct SplitGemm {
 };
 int split_gemm(const SplitGemm& g, hipStream_t st);
 
-// Planes of rows [r0, r1) x columns [c0, c1) of the fp32 matrix A (n x n,
-// pitch ld), by rows (transpose = 0: chunk row = row of A, k = column) or
+// Planes of rows [r0, r1) x columns [c0, c1) of the fp32 matrix A (n x n, or
+// n x ncols; pitch ld), by rows (transpose = 0: chunk row = row of A, k = column) or
 // transposed (chunk row = column, k = row).  r0, c0 are multiples of 128;
 // lower != 0: only 128-blocks on and below the diagonal.  Chunks are those
-// of the whole matrix.  Elements past n are zeros.  squares > 1: that many
+// of the whole matrix.  Elements past n (ncols) are zeros.  squares > 1: that many
 // such regions, `step` rows and columns apart.
 int split_planes(const float* A, int64_t n, int64_t ld, int64_t sA, int64_t r0, int64_t r1, int64_t c0, int64_t c1,
                  int transpose, int lower, const SplitPlanes& out, int64_t batch, int tag, hipStream_t st,
-                 int64_t squares = 1, int64_t step = 0);
+                 int64_t squares = 1, int64_t step = 0, int64_t ncols = -1);
 
 }  // namespace icq
