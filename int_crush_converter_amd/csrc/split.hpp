@@ -2,7 +2,8 @@
 // sum of three bf16 values x0 + x1 + x2 (8 significant bits each, rounded to
 // nearest, so 24 bits in all), and a product takes the six terms x_i y_j
 // with i + j <= 2; the dropped ones are below 2^-25 |x y|.  Used by the
-// Hessian inverse's large products (chol.hip).
+// Hessian inverse's large products (chol.hip) and the greedy search's cross
+// terms (ldlq.hip).
 //
 // Operands are split once, into planes laid out as the products read them:
 // a chunk holds 128 rows x 16 k as [plane 3][octet 2][row 128][8 k] bf16
