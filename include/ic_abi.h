@@ -187,13 +187,20 @@ int ic_sgemm(int transA, int transB, int64_t M, int64_t N, int64_t K, float alph
  * first non-positive pivot of chol(H_b) (then H_b is not a valid result and
  * the caller falls back like converter/rounding.py:19-34); info[batch+b]
  * likewise for chol(H_b^-1) in method 1.
- * workspace: ic_hessian_inverse_workspace_bytes(batch, n) bytes.
+ * workspace: ic_hessian_inverse_workspace_bytes(batch, n) bytes, of which
+ * matrices of more than 2048 rows use up to 10.5 n^2 a matrix (64 GiB in all) for split
+ * operands.  ic_hessian_inverse_sized works in any workspace from
+ * ic_hessian_inverse_min_workspace_bytes(batch, n) on: as many matrices at a
+ * time as its room has planes for, or the fp32 matrix cores without them.
  * Replaces converter/gptq.py:91-121 (_prepare_hessian, _prepare_hinv),
  * converter/rounding.py:19-34 (_invert_hessian, Cholesky branch),
  * converter/ldlq.py:64-92, 169-171, 207-209. */
 int64_t ic_hessian_inverse_workspace_bytes(int64_t batch, int64_t n);
+int64_t ic_hessian_inverse_min_workspace_bytes(int64_t batch, int64_t n);
 int ic_hessian_inverse(float* H, int64_t batch, int64_t n, float damping, int method,
                        int* info, void* workspace, void* stream);
+int ic_hessian_inverse_sized(float* H, int64_t batch, int64_t n, float damping, int method,
+                             int* info, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Damping alone, in place on `batch` dense fp32 matrices [n, n] (back to
  * back): H <- H + fp32(damping) * max(mean(diag H), 1e-6) * I, the mean
@@ -316,12 +323,17 @@ int ic_ls_scales(const int8_t* Q, const float* W, int64_t rows, int64_t cols, fl
  * Column blocks of 64 take their cross terms from one GEMM over all of err
  * (fp32 MFMA; bf16 MFMA on exactly split operands when rows and cols >= 2048
  * and cols % 512 == 0, whose planes add 6 (rows + cols) cols bytes to the
- * workspace, up to 64 GiB) plus exact in-block corrections.  workspace: ic_greedy_workspace_bytes().
+ * workspace, up to 64 GiB) plus exact in-block corrections.  workspace: ic_greedy_workspace_bytes();
+ * ic_greedy_sized takes any workspace from ic_greedy_min_workspace_bytes() on
+ * (fp32 MFMA where it has no room for the planes).
  * Replaces converter/greedy.py:487-541 (greedy_local_search_pytorch) and
  * 207-285 (greedy_local_search_triton). */
 int64_t ic_greedy_workspace_bytes(int64_t rows, int64_t cols);
+int64_t ic_greedy_min_workspace_bytes(int64_t rows, int64_t cols);
 int ic_greedy(const float* W, int8_t* Q, const float* scale, int scale_kind, const float* H, int64_t rows,
               int64_t cols, int passes, int bits, void* workspace, void* stream);
+int ic_greedy_sized(const float* W, int8_t* Q, const float* scale, int scale_kind, const float* H, int64_t rows,
+                    int64_t cols, int passes, int bits, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* The p largest eigenpairs of a symmetric positive semi-definite H [n, n]
  * (fp32): seeded subspace iteration (`iters` steps of (H + mu I) Q with

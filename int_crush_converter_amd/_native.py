@@ -50,7 +50,9 @@ _SIGS = {
     "ic_scale_status": (_i32, [_vp, _i32, _i64, _vp, _vp]),
     "ic_sgemm": (_i32, [_i32, _i32, _i64, _i64, _i64, _f32, _vp, _i64, _vp, _i64, _f32, _vp, _i64, _i32, _i32, _vp]),
     "ic_hessian_inverse_workspace_bytes": (_i64, [_i64, _i64]),
+    "ic_hessian_inverse_min_workspace_bytes": (_i64, [_i64, _i64]),
     "ic_hessian_inverse": (_i32, [_vp, _i64, _i64, _f32, _i32, _vp, _vp, _vp]),
+    "ic_hessian_inverse_sized": (_i32, [_vp, _i64, _i64, _f32, _i32, _vp, _vp, _i64, _vp]),
     "ic_cholesky": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp]),
     "ic_damp_hessian": (_i32, [_vp, _i64, _i64, _f32, _vp]),
     "ic_gram_tn": (_i32, [_vp, _i64, _i64, _i64, _f32, _vp, _vp]),
@@ -67,7 +69,9 @@ _SIGS = {
     "ic_ldlq_update_scales": (_i32, [_vp, _vp, _vp, _vp, _i64, _f32, _f32, _f32, _vp, _vp]),
     "ic_ls_scales": (_i32, [_vp, _vp, _i64, _i64, _vp, _vp]),
     "ic_greedy_workspace_bytes": (_i64, [_i64, _i64]),
+    "ic_greedy_min_workspace_bytes": (_i64, [_i64, _i64]),
     "ic_greedy": (_i32, [_vp, _vp, _vp, _i32, _vp, _i64, _i64, _i32, _i32, _vp, _vp]),
+    "ic_greedy_sized": (_i32, [_vp, _vp, _vp, _i32, _vp, _i64, _i64, _i32, _i32, _vp, _i64, _vp]),
     "ic_lowrank_workspace_bytes": (_i64, [_i64, _i64]),
     "ic_lowrank_eigs": (_i32, [_vp, _i64, _i64, _i32, _c.c_ulonglong, _f32, _vp, _vp, _c.POINTER(_i32), _vp,
                                _vp]),
@@ -241,6 +245,17 @@ def dtype_code(t: torch.Tensor) -> int:
 def workspace(nbytes: int, dev: torch.device) -> torch.Tensor:
     """Caller-owned scratch for an ABI call (uint8, through torch's allocator)."""
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=dev)
+
+
+def workspace_at_least(nbytes: int, least: int, dev: torch.device) -> torch.Tensor:
+    """``nbytes`` of scratch, or ``least`` where the GPU has no room for them
+    (for calls that are told how much they got)."""
+    try:
+        return workspace(nbytes, dev)
+    except torch.OutOfMemoryError:
+        if least >= nbytes:
+            raise
+    return workspace(least, dev)
 
 
 def row_ld(t: torch.Tensor) -> int:

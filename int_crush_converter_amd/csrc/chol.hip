@@ -1026,9 +1026,10 @@ static int64_t split_bytes(int64_t batch, int64_t n, char* base, SplitWork* w) {
     return batch * (3 * tri + rect) * (int64_t)sizeof(uint16_t);
 }
 
-// The planes take 14 n^2 bytes beside the 8 n^2 of H and X: matrices beyond
-// SPLIT_MAX_N (60 GB of planes) are inverted without them, and a batch whose
-// planes would take more than SPLIT_MAX_BYTES one matrix after the other.
+// The planes take 10.5 n^2 bytes a matrix (three triangles of 3 n^2, n^2 / 4 of
+// products at 6 bytes) beside the 8 n^2 of H and X: matrices beyond SPLIT_MAX_N
+// (45 GB of planes) are inverted without them, and a batch in pieces whose
+// planes take SPLIT_MAX_BYTES at most, or what room the workspace has.
 constexpr int64_t SPLIT_MAX_N = 65536, SPLIT_MAX_BYTES = 64LL << 30;
 // Up to SPLIT_ALIGNED_N the fp32 kernels keep up where their rows are aligned
 // (a layer with a 3072 x 3072 Hessian 4.03 ms, 4.08 split); where they are not
@@ -1037,14 +1038,22 @@ constexpr int64_t SPLIT_ALIGNED_N = 3072;
 static bool splits(int64_t n) {
     return n > (n % 4 == 0 ? SPLIT_ALIGNED_N : SPLIT_SEG) && n <= SPLIT_MAX_N;
 }
-static int64_t split_batch(int64_t batch, int64_t n) {
-    return split_bytes(batch, n, nullptr, nullptr) > SPLIT_MAX_BYTES ? 1 : batch;
+// Matrices of a batch that are inverted at once, their planes in `room` bytes
+// (0: without planes).
+static int64_t split_batch(int64_t batch, int64_t n, int64_t room) {
+    if (!splits(n)) return 0;
+    return std::min(batch, std::min(room - 256, SPLIT_MAX_BYTES) / split_bytes(1, n, nullptr, nullptr));
+}
+
+extern "C" int64_t ic_hessian_inverse_min_workspace_bytes(int64_t batch, int64_t n) {
+    return (batch * n * n + dinv_floats(batch, n)) * (int64_t)sizeof(float) +
+           dinv_floats(batch, n) * (int64_t)sizeof(double) + 256;
 }
 
 extern "C" int64_t ic_hessian_inverse_workspace_bytes(int64_t batch, int64_t n) {
-    return (batch * n * n + dinv_floats(batch, n)) * (int64_t)sizeof(float) +
-           dinv_floats(batch, n) * (int64_t)sizeof(double) + 256 +
-           (splits(n) ? split_bytes(split_batch(batch, n), n, nullptr, nullptr) + 256 : 0);
+    const int64_t step = split_batch(batch, n, INT64_MAX);
+    return ic_hessian_inverse_min_workspace_bytes(batch, n) +
+           (step > 0 ? split_bytes(step, n, nullptr, nullptr) + 256 : 0);
 }
 
 // `batch` damped matrices H -> their inverses (ic_hessian_inverse's methods);
@@ -1085,13 +1094,15 @@ static int inverse(float* H, int64_t batch, int64_t n, int method, int* info, in
     return IC_OK;
 }
 
-extern "C" int ic_hessian_inverse(float* H, int64_t batch, int64_t n, float damping, int method, int* info,
-                                  void* workspace, void* stream) {
+extern "C" int ic_hessian_inverse_sized(float* H, int64_t batch, int64_t n, float damping, int method, int* info,
+                                        void* workspace, int64_t workspace_bytes, void* stream) {
     IC_REQUIRE(H && info && workspace, "ic_hessian_inverse: null pointer");
     IC_REQUIRE(n >= 0 && batch >= 0, "ic_hessian_inverse: bad size");
     IC_REQUIRE(method >= 0 && method <= 2,
                "ic_hessian_inverse: method must be 0 (hinv), 1 (cholesky) or 2 (hinv, upper triangle)");
     if (n == 0 || batch == 0) return IC_OK;
+    const int64_t least = ic_hessian_inverse_min_workspace_bytes(batch, n);
+    IC_REQUIRE(workspace_bytes >= least, "ic_hessian_inverse: workspace too small");
     hipStream_t st = as_stream(stream);
     const int64_t sH = n * n;
     float* X = reinterpret_cast<float*>(workspace);
@@ -1100,17 +1111,25 @@ extern "C" int ic_hessian_inverse(float* H, int64_t batch, int64_t n, float damp
     IC_CHECK_HIP(hipMemsetAsync(info, 0, batch * sizeof(int), st));
     hipLaunchKernelGGL(damp_kernel, dim3((unsigned)batch), dim3(256), 0, st, H, n, n, sH, damping);
     IC_CHECK_LAUNCH();
-    if (!splits(n)) return inverse(H, batch, n, method, info, info + batch, X, dinv64, nullptr, st);
+    const int64_t step = split_batch(batch, n, workspace_bytes - least);
+    if (step <= 0) return inverse(H, batch, n, method, info, info + batch, X, dinv64, nullptr, st);
     const uintptr_t end = reinterpret_cast<uintptr_t>(dinv64 + dinv_floats(batch, n));
-    const int64_t step = split_batch(batch, n);
-    SplitWork w;
-    split_bytes(step, n, reinterpret_cast<char*>((end + 255) & ~(uintptr_t)255), &w);
+    char* planes = reinterpret_cast<char*>((end + 255) & ~(uintptr_t)255);
     for (int64_t b = 0; b < batch; b += step) {
-        int rc = inverse(H + b * sH, step, n, method, info + b, info + batch + b, X + b * sH,
+        const int64_t m = std::min(step, batch - b);
+        SplitWork w;
+        split_bytes(m, n, planes, &w);
+        int rc = inverse(H + b * sH, m, n, method, info + b, info + batch + b, X + b * sH,
                          dinv64 + dinv_floats(b, n), &w, st);
         if (rc) return rc;
     }
     return IC_OK;
+}
+
+extern "C" int ic_hessian_inverse(float* H, int64_t batch, int64_t n, float damping, int method, int* info,
+                                  void* workspace, void* stream) {
+    return ic_hessian_inverse_sized(H, batch, n, damping, method, info, workspace,
+                                    ic_hessian_inverse_workspace_bytes(batch, n), stream);
 }
 
 extern "C" int ic_damp_hessian(float* H, int64_t batch, int64_t n, float damping, void* stream) {

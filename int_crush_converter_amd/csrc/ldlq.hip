@@ -666,17 +666,22 @@ extern "C" int ic_ls_scales(const int8_t* Q, const float* W, int64_t rows, int64
     return IC_OK;
 }
 
-extern "C" int64_t ic_greedy_workspace_bytes(int64_t rows, int64_t cols) {
-    return (2 * rows * cols + rows * GSB + GSPLIT * rows * GSB) * (int64_t)sizeof(float) + 256 +
-           greedy_plane_bytes(rows, cols, nullptr, nullptr);
+extern "C" int64_t ic_greedy_min_workspace_bytes(int64_t rows, int64_t cols) {
+    return (2 * rows * cols + rows * GSB + GSPLIT * rows * GSB) * (int64_t)sizeof(float) + 256;
 }
 
-extern "C" int ic_greedy(const float* W, int8_t* Q, const float* scale, int scale_kind, const float* H, int64_t rows,
-                         int64_t cols, int passes, int bits, void* workspace, void* stream) {
+extern "C" int64_t ic_greedy_workspace_bytes(int64_t rows, int64_t cols) {
+    return ic_greedy_min_workspace_bytes(rows, cols) + greedy_plane_bytes(rows, cols, nullptr, nullptr);
+}
+
+extern "C" int ic_greedy_sized(const float* W, int8_t* Q, const float* scale, int scale_kind, const float* H,
+                               int64_t rows, int64_t cols, int passes, int bits, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
     IC_REQUIRE(W && Q && scale && H && workspace, "ic_greedy: null pointer");
     IC_REQUIRE(bits == 4 || bits == 8, "ic_greedy: bits must be 4 or 8");
     IC_REQUIRE(scale_kind == 0 || scale_kind == 1, "ic_greedy: scale_kind must be 0 (per row) or 1 (per element)");
     if (rows == 0 || cols == 0 || passes <= 0) return IC_OK;
+    IC_REQUIRE(workspace_bytes >= ic_greedy_min_workspace_bytes(rows, cols), "ic_greedy: workspace too small");
     hipStream_t st = as_stream(stream);
     const float qmin = bits == 4 ? -8.0f : -128.0f, qmax = bits == 4 ? 7.0f : 127.0f;
     float* err = reinterpret_cast<float*>(workspace);
@@ -687,7 +692,8 @@ extern "C" int ic_greedy(const float* W, int8_t* Q, const float* scale, int scal
     IC_CHECK_LAUNCH();
     float* part = cross + rows * GSB;
     GreedyPlanes planes, *pl = nullptr;
-    if (passes > 0 && greedy_plane_bytes(rows, cols, reinterpret_cast<char*>(part + GSPLIT * rows * GSB), &planes)) {
+    if (workspace_bytes >= ic_greedy_workspace_bytes(rows, cols) &&
+        greedy_plane_bytes(rows, cols, reinterpret_cast<char*>(part + GSPLIT * rows * GSB), &planes)) {
         pl = &planes;
         int rc = split_planes(H, cols, cols, 0, 0, cols, 0, cols, 0, 0, pl->H, 1, PT_GEMM_GREEDY, st);
         if (!rc)
@@ -701,6 +707,12 @@ extern "C" int ic_greedy(const float* W, int8_t* Q, const float* scale, int scal
     hipLaunchKernelGGL(to_int8_kernel, dim3(egrid(rows * cols)), dim3(256), 0, st, Qf, rows * cols, qmin, qmax, Q);
     IC_CHECK_LAUNCH();
     return IC_OK;
+}
+
+extern "C" int ic_greedy(const float* W, int8_t* Q, const float* scale, int scale_kind, const float* H, int64_t rows,
+                         int64_t cols, int passes, int bits, void* workspace, void* stream) {
+    return ic_greedy_sized(W, Q, scale, scale_kind, H, rows, cols, passes, bits, workspace,
+                           ic_greedy_workspace_bytes(rows, cols), stream);
 }
 
 extern "C" int64_t ic_greedy_lowrank_workspace_bytes(int64_t rows, int64_t cols, int64_t k) {

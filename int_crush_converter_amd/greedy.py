@@ -81,8 +81,10 @@ def greedy_local_search(W, Q, scale, H, num_passes: int, clamp_min: int, clamp_m
     Wg, Qg, s, kind, Hg = _prep(W, Q, scale, H)
     M, N = Wg.shape
     Qo = Qg.clone()
-    ws = nat.workspace(_lib().ic_greedy_workspace_bytes(M, N), Wg.device)
-    nat.check(_lib().ic_greedy(Wg, Qo, s, kind, Hg, M, N, int(num_passes), bits, ws, nat.stream()), "ic_greedy")
+    ws = nat.workspace_at_least(_lib().ic_greedy_workspace_bytes(M, N), _lib().ic_greedy_min_workspace_bytes(M, N),
+                                Wg.device)
+    nat.check(_lib().ic_greedy_sized(Wg, Qo, s, kind, Hg, M, N, int(num_passes), bits, ws, ws.numel(), nat.stream()),
+              "ic_greedy")
     return Qo.to(W.device)
 
 

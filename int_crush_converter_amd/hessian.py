@@ -70,9 +70,10 @@ def inverse_batch(H: torch.Tensor, damping: float, method: str = "hinv",
     if upper_only and code == 0:
         code = 2
     info = torch.zeros(2 * batch, dtype=torch.int32, device=out.device)
-    ws = nat.workspace(nat.lib().ic_hessian_inverse_workspace_bytes(batch, n), out.device)
-    nat.check(nat.lib().ic_hessian_inverse(out, batch, n, float(damping), code, info,
-                                           ws, nat.stream()), "ic_hessian_inverse")
+    ws = nat.workspace_at_least(nat.lib().ic_hessian_inverse_workspace_bytes(batch, n),
+                                nat.lib().ic_hessian_inverse_min_workspace_bytes(batch, n), out.device)
+    nat.check(nat.lib().ic_hessian_inverse_sized(out, batch, n, float(damping), code, info, ws, ws.numel(),
+                                                 nat.stream()), "ic_hessian_inverse")
     del ws
     inf = info.tolist()
     orig = None
