@@ -616,7 +616,9 @@ extern "C" int ic_lowrank_eigs(const float* H, int64_t n, int64_t p, int iters, 
     LrWork w;
     char* base = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(workspace) + 255) & ~(uintptr_t)255);
     lr_layout(n, p, base, &w);
-    IC_CHECK_HIP(hipMemsetAsync(w.info, 0, 2 * sizeof(int), st));
+    // info[0]: the orthonormalisations; info[1 + i]: the certificate's i-th test
+    // (a factorisation reports a bad pivot only where none is reported yet)
+    IC_CHECK_HIP(hipMemsetAsync(w.info, 0, 3 * sizeof(int), st));
     const int64_t np = n * p;
     // mu = 1e-3 lambda_max estimate (power iteration from a seeded vector)
     constexpr int POWER_STEPS = 16;
@@ -653,9 +655,10 @@ extern "C" int ic_lowrank_eigs(const float* H, int64_t n, int64_t p, int iters, 
             hipLaunchKernelGGL(sub_frob_diag_kernel, dim3(1), dim3(256), 0, st, w.T, p, w.part, LR_PARTS,
                                (double)refuse_rel);
             IC_CHECK_LAUNCH();
-            if ((rc = potrf(w.T, 1, p, p, p * p, w.dinv64, w.info + 1, st))) return rc;
+            int* test_info = w.info + 1 + (it - test_lo);
+            if ((rc = potrf(w.T, 1, p, p, p * p, w.dinv64, test_info, st))) return rc;
             int pd_info = 0;
-            IC_CHECK_HIP(hipMemcpyAsync(&pd_info, w.info + 1, sizeof(int), hipMemcpyDeviceToHost, st));
+            IC_CHECK_HIP(hipMemcpyAsync(&pd_info, test_info, sizeof(int), hipMemcpyDeviceToHost, st));
             IC_CHECK_HIP(hipStreamSynchronize(st));
             if (pd_info == 0) {
                 if (sweeps_out) *sweeps_out = 0;
