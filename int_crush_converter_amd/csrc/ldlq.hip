@@ -8,7 +8,7 @@
 // and the changes d_j' of earlier columns of the block are added exactly as
 // sum_j' d_j' H[j', j] - the same quantity in exact arithmetic as the
 // reference's per-column GEMV (its fp32 rounding differs).
-#include "gemm.hpp"
+#include "gemm_dev.hpp"
 #include "split.hpp"
 #include "torchsum.hpp"
 
@@ -499,11 +499,8 @@ constexpr int PROXY_PARTS = 1024;
 constexpr int GSPLIT = 4;
 
 // C[r][c] = ((P_0 + P_1) + P_2) + P_3 for the GSPLIT partial products
-// (pitch GSB, stride rows * GSB).  err (or null): P came from split operands,
-// where an infinity gives a NaN; such sums are formed again in fp32 from err's
-// and Hsb's rows (pitch cols), so that a NaN here is one of theirs.
-__global__ void split_sum_kernel(const float* __restrict__ P, int64_t rows, int64_t sw, float* __restrict__ C,
-                                 const float* __restrict__ err, const float* __restrict__ Hsb, int64_t cols) {
+// (pitch GSB, stride rows * GSB).
+__global__ void split_sum_kernel(const float* __restrict__ P, int64_t rows, int64_t sw, float* __restrict__ C) {
     const int64_t total = rows * sw, stride = rows * GSB;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
          i += (int64_t)gridDim.x * blockDim.x) {
@@ -511,11 +508,38 @@ __global__ void split_sum_kernel(const float* __restrict__ P, int64_t rows, int6
         float v = P[o];
 #pragma unroll
         for (int k = 1; k < GSPLIT; ++k) v = v + P[k * stride + o];
-        if (err && !(fabsf(v) <= 3.402823466e38f)) {
-            v = 0.0f;
-            for (int64_t j = 0; j < cols; ++j) v = __builtin_fmaf(err[r * cols + j], Hsb[c * cols + j], v);
-        }
         C[o] = v;
+    }
+}
+
+// The same sums of products of split operands, where an infinity gives a NaN:
+// a 64 x 64 tile (a work-group) with a sum that is not finite is formed again
+// as the fp32 product g, in place of P_0, and such sums are taken from there,
+// so that a NaN in C is one of theirs.  (One infinity in every row, [2050,
+// 2048], one pass: 7.3 ms, 35.7 with one thread summing the K products of such
+// an element; 4.3 without infinities.  [4096, 4096]: 15.8 and 8.2 ms.)
+__global__ __launch_bounds__(256) void split_sum_checked_kernel(const float* P, int64_t rows, int64_t sw, float* C,
+                                                               GemmArgs g) {
+    __shared__ __attribute__((aligned(16))) float lds[2 * gk::Geo<64>::TILE_F];
+    const int64_t stride = rows * GSB, r0 = (int64_t)blockIdx.y * 64, c = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    auto finite = [](float v) { return fabsf(v) <= 3.402823466e38f; };
+    bool bad = false;
+#pragma unroll 4
+    for (int u = 0; u < 16; ++u) {
+        const int64_t r = r0 + 4 * u + (threadIdx.x >> 6), o = r * GSB + c;
+        if (r >= rows || c >= sw) continue;
+        float v = P[o];
+#pragma unroll
+        for (int k = 1; k < GSPLIT; ++k) v = v + P[k * stride + o];
+        C[o] = v;
+        bad |= !finite(v);
+    }
+    if (!__syncthreads_or(bad)) return;   // (every thread has read its part of P_0)
+    gk::gemm_tile<0, 1, true, 64, gk::CHUNK_SUM>(g, gk::tile_range<64>(g, blockIdx.y, blockIdx.x), 0, lds);
+    __syncthreads();
+    for (int u = 0; u < 16; ++u) {
+        const int64_t r = r0 + 4 * u + (threadIdx.x >> 6), o = r * GSB + c;
+        if (r < rows && c < sw && !finite(C[o])) C[o] = P[o];
     }
 }
 
@@ -575,16 +599,17 @@ static int greedy_pass(float* err, float* Qf, const float* sc, int pe, const flo
             g.tag = PT_GEMM_GREEDY;
             g.algo_flops = 2.0 * rows * sw * cols;
             if ((rc = split_gemm(g, st))) return rc;
-            hipLaunchKernelGGL(split_sum_kernel, dim3(egrid(rows * sw)), dim3(256), 0, st, part, rows, sw, C, err,
-                               Hc + s0 * cols, cols);
+            const GemmArgs f{rows, sw, cols, 1.0f, 0.0f, err, cols, 0, Hc + s0 * cols, cols, 0, part, GSB, 0, 0, 1,
+                             CMASK_FULL, KR_FULL, 1, PT_GEMM_GREEDY};
+            hipLaunchKernelGGL(split_sum_checked_kernel, dim3((unsigned)cdiv(sw, 64), (unsigned)cdiv(rows, 64)),
+                               dim3(256), 0, st, part, rows, sw, C, f);
             IC_CHECK_LAUNCH();
         } else if (split) {
             GemmArgs g{rows, sw, ks, 1.0f, 0.0f, err, cols, ks, Hc + s0 * cols, cols, ks, part, GSB, rows * GSB,
                        0, 1, CMASK_FULL, KR_FULL, GSPLIT, PT_GEMM_GREEDY};
             g.algo_flops = 2.0 * rows * sw * cols;
             if ((rc = gemm_f32(g, st))) return rc;
-            hipLaunchKernelGGL(split_sum_kernel, dim3(egrid(rows * sw)), dim3(256), 0, st, part, rows, sw, C,
-                               nullptr, nullptr, 0);
+            hipLaunchKernelGGL(split_sum_kernel, dim3(egrid(rows * sw)), dim3(256), 0, st, part, rows, sw, C);
             IC_CHECK_LAUNCH();
         } else {
             GemmArgs g{rows, sw, cols, 1.0f, 0.0f, err, cols, 0, Hc + s0 * cols, cols, 0, C, GSB, 0, 0, 1,
