@@ -483,10 +483,13 @@ int ic_hbm_stream(int kind, const void* src, void* dst, int64_t bytes, void* str
  * cross-term GEMMs, 11 Cholesky panel solve, 12 RTN scales / clip search,
  * 13 fp64 verification, 14 PermuQuant (moments, sort, error scales,
  * gathers), 15 PermuQuant ordered error sums, 16 DLR r x r products,
- * 17 DLR n x n product, 18 PiSO scale search.  Enabling resets the record.
+ * 17 DLR n x n product, 18 PiSO scale search; on split operands: 19 Cholesky
+ * products, 20 inverse products, 21 greedy cross terms, 22 the splitting.
+ * Enabling resets the record.
  * ic_profile_read synchronises the events and returns, per phase, the summed
  * kernel time (ms), algorithmic flops and bytes, and the launch count (arrays
- * of at least 19 entries). */
+ * of 23 entries; with 19 to 22 a phase past the last is counted in 1, 2, 10
+ * and 9 in the order of 19 to 22). */
 int ic_profile_enable(int on);
 int ic_profile_read(double* ms, double* flops, double* bytes, int64_t* launches, int ntags);
 

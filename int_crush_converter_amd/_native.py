@@ -99,21 +99,24 @@ _SIGS = {
 
 PROFILE_TAGS = ["gemm_trailing", "gemm_cholesky", "gemm_inverse", "diag_factor", "sweep", "rotate_w",
                 "rotate_h", "rtn_quant_pack", "greedy", "other", "gemm_greedy", "chol_panel", "rtn_scales",
-                "verify", "permute", "permute_sum", "dlr", "dlr_gemm", "piso"]
+                "verify", "permute", "permute_sum", "dlr", "dlr_gemm", "piso", "split_cholesky", "split_inverse",
+                "split_greedy", "split_planes"]
 
 # kernel family -> (the profiler phases its launches are tagged with, the
-# bound it is graded against: "mfma", "hbm", or "latency" for kernels whose
-# time is a dependency chain / instruction issue, reported as a share of the
-# step).  The rotation phases are MFMA-bound with the exact kernels (the
+# bound it is graded against: "mfma" (fp32), "mfma_split" (fp32 products as six
+# bf16 ones), "hbm", or "latency" for kernels whose time is a dependency chain
+# / instruction issue, reported as a share of the step).  The rotation phases are MFMA-bound with the exact kernels (the
 # default) and HBM-bound with the fast Walsh-Hadamard transform.
 PROFILE_KERNELS = {
     "gemm_f32_kernel": (["gemm_trailing", "gemm_cholesky", "gemm_inverse", "gemm_greedy", "dlr", "dlr_gemm"], "mfma"),
-    "potrf_diag_kernel": (["diag_factor"], "latency"),
-    "panel64_kernel": (["chol_panel"], "latency"),
+    "split_gemm_kernel": (["split_cholesky", "split_inverse", "split_greedy"], "mfma_split"),
+    "split_planes_kernel": (["split_planes"], "hbm"),
+    "potrf_diag_rest_kernel / potrf_diag_kernel": (["diag_factor"], "latency"),
+    "panel_solve_kernel": (["chol_panel"], "latency"),
     "sweep16_kernel / sweep4_kernel": (["sweep"], "latency"),
     "greedy_sb_kernel": (["greedy"], "latency"),
-    "rot_rows_wave_kernel / rot_rows_exact_kernel": (["rotate_w"], "mfma"),
-    "rot_cols_exact_kernel + rot_rows_exact_kernel": (["rotate_h"], "mfma"),
+    "rot_rows_wave_kernel / rot_rows_exact_kernel": (["rotate_w"], "mfma"),          # (small launches: the
+    "rot_cols_exact_kernel + rot_rows_exact_kernel": (["rotate_h"], "mfma"),         # narrow kernels)
     "rtn_clip_reg_kernel / rtn_clip_kernel": (["rtn_scales"], "latency"),   # VALU-bound: a share of the step
     "rtn_quant_kernel": (["rtn_quant_pack"], "hbm"),
     "quant_error_partial": (["verify"], "hbm"),

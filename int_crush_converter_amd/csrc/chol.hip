@@ -840,7 +840,7 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
             if (Lp) {
                 // the rows that this update or a merge reads
                 const int64_t r = split ? s1 : cdiv(s1, SPLIT_SEG) * SPLIT_SEG;
-                int rc = split_planes(H, n, ld, sH, r, n, s0, s1, 0, 0, *Lp, batch, PT_GEMM_CHOL, st);
+                int rc = split_planes(H, n, ld, sH, r, n, s0, s1, 0, 0, *Lp, batch, st);
                 if (rc) return rc;
             }
             if (split) {
@@ -850,7 +850,7 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
                 a.c0 = s0 / SP_K;
                 a.zp = Lp->stride;
                 SplitGemm g{m, m, k, -1.0f, 1, a, a, H + s1 * ld + s1, ld, sH, SplitOp{}, CMASK_LOWER, KR_FULL, batch,
-                            PT_GEMM_CHOL, (double)batch * 2.0 * dtri((double)m) * k};
+                            PT_SPLIT_CHOL, (double)batch * 2.0 * dtri((double)m) * k};
                 int rc = split_gemm(g, st);
                 if (rc) return rc;
                 continue;
@@ -930,8 +930,8 @@ static int merge_pairs_split(float* X, int64_t n, int64_t ld, int64_t r0, int64_
     SplitPlanes T = w.T;
     T.nb = n2p / SP_K;
     const int64_t tz = pairs_batched ? n1 / SP_ROWS * T.nb * SP_CHUNK : T.stride;
-    int rc0 = split_planes(X, n, ld, sH, r0 + n1, r0 + n1 + n2, r0 + n1, r0 + n1 + n2, 0, 1, w.XR, batch, PT_GEMM_INV,
-                           st, count, count > 1 ? n1 + n2 : 0);
+    int rc0 = split_planes(X, n, ld, sH, r0 + n1, r0 + n1 + n2, r0 + n1, r0 + n1 + n2, 0, 1, w.XR, batch, st,
+                           count, count > 1 ? n1 + n2 : 0);
     if (rc0) return rc0;
     for (int64_t m = 0; m < outer; ++m) {
         const int64_t off = pairs_batched ? m : 0;
@@ -952,11 +952,11 @@ static int merge_pairs_split(float* X, int64_t n, int64_t ld, int64_t r0, int64_
         int rc;
         // T = L21 X11 (k >= column: X11 is lower)
         SplitGemm g1{n2, n1, n1, 1.0f, 0, op(w.L, b1, b0), op(w.XT, b0, b0), nullptr, 0, 0, t, CMASK_FULL, KR_FROM_J,
-                     gb, PT_GEMM_INV, (double)gb * n2 * n1 * (n1 + 1)};
+                     gb, PT_SPLIT_INV, (double)gb * n2 * n1 * (n1 + 1)};
         if ((rc = split_gemm(g1, st))) return rc;
         // X21 = -X22 T (k <= row: X22 is lower)
         SplitGemm g2{n2, n1, n2p, -1.0f, 0, op(w.XR, b1, b1), t, X + off * sH + (r0 + n1) * ld + r0, ld,
-                     pairs_batched ? step * (ld + 1) : sH, op(w.XT, b0, b1), CMASK_FULL, KR_TO_I, gb, PT_GEMM_INV,
+                     pairs_batched ? step * (ld + 1) : sH, op(w.XT, b0, b1), CMASK_FULL, KR_TO_I, gb, PT_SPLIT_INV,
                      (double)gb * n1 * n2 * (n2 + 1)};
         if ((rc = split_gemm(g2, st))) return rc;
     }
@@ -977,7 +977,7 @@ int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_
     bool split = false;   // the segments' planes exist
     while (seg.size() > 2) {
         if (w && !split && seg[1] == SPLIT_SEG) {
-            int rc = split_planes(X, n, ld, sH, 0, seg[1], 0, seg[1], 1, 1, w->XT, batch, PT_GEMM_INV, st,
+            int rc = split_planes(X, n, ld, sH, 0, seg[1], 0, seg[1], 1, 1, w->XT, batch, st,
                                   (int64_t)seg.size() - 1, seg[1]);
             if (rc) return rc;
             split = true;
@@ -1073,7 +1073,7 @@ static int inverse(float* H, int64_t batch, int64_t n, int method, int* info, in
         x.s = w->XT;
         x.zp = w->XT.stride;
         SplitGemm u{n, n, cdiv(n, SP_ROWS) * SP_ROWS, 1.0f, 0, x, x, H, ld, sH, SplitOp{}, CMASK_UPPER, KR_FROM_MAXIJ,
-                    batch, PT_GEMM_INV, flops};
+                    batch, PT_SPLIT_INV, flops};
         rc = split_gemm(u, st);
     } else {
         GemmArgs u{n, n, n, 1.0f, 0.0f, X, ld, sH, X, ld, sH, H, ld, sH, 1, 0, CMASK_UPPER, KR_FROM_MAXIJ, batch,

@@ -596,7 +596,7 @@ static int greedy_pass(float* err, float* Qf, const float* sc, int pe, const flo
             g.cmask = CMASK_FULL;
             g.krange = KR_FULL;
             g.batch = GSPLIT;
-            g.tag = PT_GEMM_GREEDY;
+            g.tag = PT_SPLIT_GREEDY;
             g.algo_flops = 2.0 * rows * sw * cols;
             if ((rc = split_gemm(g, st))) return rc;
             const GemmArgs f{rows, sw, cols, 1.0f, 0.0f, err, cols, 0, Hc + s0 * cols, cols, 0, part, GSB, 0, 0, 1,
@@ -630,7 +630,7 @@ static int greedy_pass(float* err, float* Qf, const float* sc, int pe, const flo
             IC_CHECK_LAUNCH();
         }
         if (pl) {   // the columns that changed
-            int rc2 = split_planes(err, rows, cols, 0, 0, rows, s0, s0 + sw, 0, 0, pl->E, 1, PT_GEMM_GREEDY, st, 1, 0,
+            int rc2 = split_planes(err, rows, cols, 0, 0, rows, s0, s0 + sw, 0, 0, pl->E, 1, st, 1, 0,
                                    cols);
             if (rc2) return rc2;
         }
@@ -720,9 +720,9 @@ extern "C" int ic_greedy_sized(const float* W, int8_t* Q, const float* scale, in
     if (workspace_bytes >= ic_greedy_workspace_bytes(rows, cols) &&
         greedy_plane_bytes(rows, cols, reinterpret_cast<char*>(part + GSPLIT * rows * GSB), &planes)) {
         pl = &planes;
-        int rc = split_planes(H, cols, cols, 0, 0, cols, 0, cols, 0, 0, pl->H, 1, PT_GEMM_GREEDY, st);
+        int rc = split_planes(H, cols, cols, 0, 0, cols, 0, cols, 0, 0, pl->H, 1, st);
         if (!rc)
-            rc = split_planes(err, rows, cols, 0, 0, rows, 0, cols, 0, 0, pl->E, 1, PT_GEMM_GREEDY, st, 1, 0, cols);
+            rc = split_planes(err, rows, cols, 0, 0, rows, 0, cols, 0, 0, pl->E, 1, st, 1, 0, cols);
         if (rc) return rc;
     }
     for (int p = 0; p < passes; ++p) {

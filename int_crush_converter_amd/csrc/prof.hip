@@ -57,7 +57,10 @@ extern "C" int ic_profile_enable(int on) {
 }
 
 extern "C" int ic_profile_read(double* ms, double* flops, double* bytes, int64_t* launches, int ntags) {
-    IC_REQUIRE(ms && flops && bytes && launches && ntags >= PT_COUNT, "ic_profile_read: need PT_COUNT slots");
+    // (19: the phases without those of split operands, which then count with the phase they are part of)
+    IC_REQUIRE(ms && flops && bytes && launches && ntags >= PT_SPLIT_CHOL, "ic_profile_read: need 19 slots");
+    static_assert(PT_COUNT == PT_SPLIT_CHOL + 4, "a phase for each below");
+    constexpr int part_of[] = {PT_GEMM_CHOL, PT_GEMM_INV, PT_GEMM_GREEDY, PT_OTHER};
     std::lock_guard<std::mutex> lk(g_mu);
     for (int t = 0; t < ntags; ++t) { ms[t] = 0; flops[t] = 0; bytes[t] = 0; launches[t] = 0; }
     for (size_t i = 0; i < g_used; ++i) {
@@ -65,10 +68,11 @@ extern "C" int ic_profile_read(double* ms, double* flops, double* bytes, int64_t
         IC_CHECK_HIP(hipEventSynchronize(r.b));
         float e = 0.0f;
         IC_CHECK_HIP(hipEventElapsedTime(&e, r.a, r.b));
-        ms[r.tag] += e;
-        flops[r.tag] += r.flops;
-        bytes[r.tag] += r.bytes;
-        launches[r.tag] += 1;
+        const int t = r.tag < ntags ? r.tag : part_of[r.tag - PT_SPLIT_CHOL];
+        ms[t] += e;
+        flops[t] += r.flops;
+        bytes[t] += r.bytes;
+        launches[t] += 1;
     }
     return IC_OK;
 }

@@ -29,7 +29,11 @@ enum ProfTag : int {
     PT_DLR = 16,         // Woodbury inverse: r x r products
     PT_DLR_GEMM = 17,    // Woodbury / dense DLR: the n x n product
     PT_PISO = 18,        // PiSO scale search
-    PT_COUNT = 19,
+    PT_SPLIT_CHOL = 19,  // potrf SYRK from split operands (split_gemm)
+    PT_SPLIT_INV = 20,   // trtri + lauum from split operands
+    PT_SPLIT_GREEDY = 21,  // greedy cross terms from split operands
+    PT_SPLIT_PLANES = 22,  // operands split into planes
+    PT_COUNT = 23,
 };
 
 bool prof_enabled();

@@ -342,14 +342,14 @@ int split_gemm(const SplitGemm& g, hipStream_t st) {
 }
 
 int split_planes(const float* A, int64_t n, int64_t ld, int64_t sA, int64_t r0, int64_t r1, int64_t c0, int64_t c1,
-                 int transpose, int lower, const SplitPlanes& out, int64_t batch, int tag, hipStream_t st,
-                 int64_t squares, int64_t step, int64_t ncols) {
+                 int transpose, int lower, const SplitPlanes& out, int64_t batch, hipStream_t st, int64_t squares,
+                 int64_t step, int64_t ncols) {
     if (r1 <= r0 || c1 <= c0 || batch <= 0) return IC_OK;
     IC_REQUIRE(r0 % SP_ROWS == 0 && c0 % SP_ROWS == 0, "split_planes: unaligned block");
     const int64_t rbs = cdiv(r1 - r0, SP_ROWS), cbs = cdiv(c1 - c0, SP_ROWS);
     IC_REQUIRE(step % SP_ROWS == 0 && rbs <= 65535 && batch * squares <= 65535, "split_planes: problem too large");
     const bool vec = ((uintptr_t)A % 16) == 0 && ld % 4 == 0 && sA % 4 == 0;
-    ProfScope prof_scope(st, tag, 0.0, 10.0 * batch * squares * (r1 - r0) * (c1 - c0));
+    ProfScope prof_scope(st, PT_SPLIT_PLANES, 0.0, 10.0 * batch * squares * (r1 - r0) * (c1 - c0));
     const dim3 gd((unsigned)cbs, (unsigned)rbs, (unsigned)(batch * squares));
     const int64_t rb0 = r0 / SP_ROWS, cb0 = c0 / SP_ROWS;
     if (ncols < 0) ncols = n;

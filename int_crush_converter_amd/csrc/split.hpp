@@ -71,7 +71,7 @@ int split_gemm(const SplitGemm& g, hipStream_t st);
 // of the whole matrix.  Elements past n (ncols) are zeros.  squares > 1: that many
 // such regions, `step` rows and columns apart.
 int split_planes(const float* A, int64_t n, int64_t ld, int64_t sA, int64_t r0, int64_t r1, int64_t c0, int64_t c1,
-                 int transpose, int lower, const SplitPlanes& out, int64_t batch, int tag, hipStream_t st,
-                 int64_t squares = 1, int64_t step = 0, int64_t ncols = -1);
+                 int transpose, int lower, const SplitPlanes& out, int64_t batch, hipStream_t st, int64_t squares = 1,
+                 int64_t step = 0, int64_t ncols = -1);
 
 }  // namespace icq
