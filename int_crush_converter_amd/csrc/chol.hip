@@ -768,7 +768,7 @@ constexpr int64_t SPLIT_SEG = 2048;
 constexpr int64_t SPLIT_SYRK_BLOCKS = 15;
 
 int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* dinv64, int* info, hipStream_t st,
-          const SplitPlanes* Lp) {
+          const SplitPlanes* Lp, bool merges) {
     const int64_t nblk = cdiv(n, NB);
     const int64_t dstride = nblk * NB * NB;
     IC_REQUIRE(batch <= 65535, "potrf: batch too large");
@@ -837,7 +837,7 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
             const float* P = H + s1 * ld + s0;
             const int64_t k = s1 - s0;
             const bool split = Lp && cdiv(m, SP_ROWS) >= SPLIT_SYRK_BLOCKS;
-            if (Lp) {
+            if (split || (Lp && merges)) {
                 // the rows that this update or a merge reads
                 const int64_t r = split ? s1 : cdiv(s1, SPLIT_SEG) * SPLIT_SEG;
                 int rc = split_planes(H, n, ld, sH, r, n, s0, s1, 0, 0, *Lp, batch, st);
@@ -1062,7 +1062,7 @@ static int inverse(float* H, int64_t batch, int64_t n, int method, int* info, in
                    const SplitWork* w, hipStream_t st) {
     const int64_t ld = n, sH = n * n;
     const SplitPlanes* Lp = w ? &w->L : nullptr;
-    int rc = potrf(H, batch, n, ld, sH, dinv64, info, st, Lp);
+    int rc = potrf(H, batch, n, ld, sH, dinv64, info, st, Lp, true);
     if (rc) return rc;
     rc = trtri(H, X, batch, n, ld, sH, dinv64, st, w);
     if (rc) return rc;
@@ -1085,7 +1085,7 @@ static int inverse(float* H, int64_t batch, int64_t n, int method, int* info, in
     if ((rc = mirror_upper(H, batch, n, ld, sH, st))) return rc;
     if (method == 1) {
         // upper Cholesky factor of H^-1 (converter/gptq.py:91-110): L2 = chol(H^-1), return L2^T
-        rc = potrf(H, batch, n, ld, sH, dinv64, info2, st, Lp);
+        rc = potrf(H, batch, n, ld, sH, dinv64, info2, st, Lp, false);
         if (rc) return rc;
         dim3 tb(16, 16), tg((unsigned)cdiv(n, 16), (unsigned)cdiv(n, 16), (unsigned)batch);
         hipLaunchKernelGGL(lower_to_upper_kernel, tg, tb, 0, st, H, n, ld, sH);

@@ -16,10 +16,11 @@ double* dinv64_of(float* dinv, int64_t batch, int64_t n);
 // info[b] receives the 1-based column of the first non-positive pivot (or
 // stays as it was).  The strict upper triangle is left as it was, except in
 // the 128 x 128 diagonal blocks (zeroed).
-// Lp: planes for L (SP_LOWER); they then hold the blocks that trtri's split
-// merges read, and the larger trailing updates are split products.
+// Lp: planes for L (SP_LOWER): the larger trailing updates are split products,
+// and with `merges` the planes then hold the blocks that trtri's split merges
+// read.
 int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* dinv64, int* info, hipStream_t st,
-          const SplitPlanes* Lp = nullptr);
+          const SplitPlanes* Lp = nullptr, bool merges = false);
 
 // Split planes of a large inverse: L (from potrf), X^T (whole on return), X
 // by rows and the merges' intermediate products.

@@ -55,3 +55,21 @@ def test_split_products_have_their_own_phases(gpu_dev):
         assert la[nat.PROFILE_TAGS.index(whole)] == prof[split]["launches"] + prof[whole]["launches"]
     name, roof = bench.roofline_from(prof, "")
     assert 0 < roof["frac"] < 1, (name, roof)
+
+
+@pytest.mark.gpu
+def test_planes_that_nothing_reads_are_not_formed(gpu_dev):
+    # n = 3200: columns 1024 .. 2047 have an update of 1152 rows, which is not split, below them; a merge reads their
+    # planes.  chol(H^-1) has no merge: one set of planes, for the split update of 2176 rows
+    from int_crush_converter_amd.hessian import inverse_batch
+    from tests.conftest import lognormal_hessian
+    H = lognormal_hessian(3200, 3712, 1).to(gpu_dev)
+    launches = {}
+    for method in ("hinv", "cholesky"):
+        nat.profile_enable(True)
+        try:
+            inverse_batch(H, 0.01, method)
+            launches[method] = nat.profile_read()["split_planes"]["launches"]
+        finally:
+            nat.profile_enable(False)
+    assert launches["cholesky"] == launches["hinv"] + 1, launches
