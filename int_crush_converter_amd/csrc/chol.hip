@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void damp_kernel(float* H, int64_t n, int64_t 
 
 // Factor the diagonal block [k0, k0+nb) of a matrix in place (lower, upper
 // part of the block set to 0) and write what the panel solve and the
-// triangular inverse need of it to dinv64 (packed tiles, below).  info[b]
+// triangular inverse need of it to `tiles` (packed, below).  info[b]
 // gets the 1-based column of the first non-positive pivot (LAPACK convention)
 // if it is still 0.  A partial block (nb < 128) is padded with the identity.
 //
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256) void damp_kernel(float* H, int64_t n, int64_t 
 //   D (4 doubles v): D[i = l/16 + 4*v][j = l%16]
 // so a D fragment is the B operand of four MFMA steps as it stands.
 //
-// Packed tiles: tile (J, K), K <= J, of a block's factor at dinv64 +
+// Packed tiles: tile (J, K), K <= J, of a block's factor at tiles +
 // (J (J + 1) / 2 + K) * 256, in A-operand order with two steps adjacent:
 // value [h][lane][e] is L[16 J + perm16(l%16)][16 K + 4 (l/16) + 2 h + e], and on the
 // diagonal the same of L_JJ^-1.  perm16 orders the 16 indices so that the four
@@ -437,9 +437,9 @@ __device__ __forceinline__ void diag_factor_wave(DiagShared& sh, float* A, int64
 // are 16-byte aligned).
 template <bool UPD, bool VEC = false>
 __device__ __forceinline__ void diag_block(DiagShared& sh, int b, float* H, int64_t ld, int64_t stride, int64_t k0,
-                                           int nb, double* dinv64, int64_t dstride, int* info) {
+                                           int nb, double* tiles, int64_t dstride, int* info) {
     float* A = H + (int64_t)b * stride + k0 * ld + k0;
-    double* packed = dinv64 + (int64_t)b * dstride;
+    double* packed = tiles + (int64_t)b * dstride;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform
     int bad = 0;
@@ -482,10 +482,10 @@ __device__ __forceinline__ void diag_block(DiagShared& sh, int b, float* H, int6
 }
 
 __global__ __launch_bounds__(DIAG_WAVES * 64) void potrf_diag_kernel(float* H, int64_t ld, int64_t stride, int64_t k0,
-                                                                    int nb, double* dinv64, int64_t dstride,
+                                                                    int nb, double* tiles, int64_t dstride,
                                                                     int* info) {
     __shared__ __attribute__((aligned(16))) DiagShared sh;
-    diag_block<false>(sh, blockIdx.x, H, ld, stride, k0, nb, dinv64, dstride, info);
+    diag_block<false>(sh, blockIdx.x, H, ld, stride, k0, nb, tiles, dstride, info);
 }
 
 // The diagonal block of matrix blockIdx.z (work-group 0), which it updates
@@ -500,11 +500,11 @@ constexpr int REST_T = 128;
 static_assert(2 * gk::Geo<REST_T>::TILE_F * sizeof(float) <= sizeof(DiagShared), "GEMM tile staging fits");
 template <bool VEC>
 __global__ __launch_bounds__(DIAG_WAVES * 64) void potrf_diag_rest_kernel(float* H, int64_t ld, int64_t stride,
-                                                                         int64_t k0, int nb, double* dinv64,
+                                                                         int64_t k0, int nb, double* tiles,
                                                                          int64_t dstride, int* info, GemmArgs g) {
     __shared__ __attribute__((aligned(16))) DiagShared sh;
     if (blockIdx.x == 0) {
-        diag_block<true, VEC>(sh, blockIdx.z, H, ld, stride, k0, nb, dinv64, dstride, info);
+        diag_block<true, VEC>(sh, blockIdx.z, H, ld, stride, k0, nb, tiles, dstride, info);
         return;
     }
     if (threadIdx.x >= 256) return;
@@ -606,10 +606,10 @@ __device__ __forceinline__ void panel_wave(float* P, int64_t m, int64_t ld, cons
 
 template <bool VEC>
 __global__ __launch_bounds__(256) void panel_solve_kernel(float* A21, int64_t m, int64_t ld, int64_t stride,
-                                                         const double* dinv64, int64_t dstride, int groups) {
+                                                         const double* tiles, int64_t dstride, int groups) {
     __shared__ double xs[2][4][64];
     float* P = A21 + (int64_t)blockIdx.y * stride;
-    const double* packed = dinv64 + (int64_t)blockIdx.y * dstride;
+    const double* packed = tiles + (int64_t)blockIdx.y * dstride;
     const int lane = threadIdx.x & 63;
     switch (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {
         case 0: panel_wave<0, VEC>(P, m, ld, packed, groups, xs, lane); break;
@@ -671,9 +671,9 @@ __device__ __forceinline__ void dinv_wave(float* P, int64_t ld, int nb, const do
 }
 
 __global__ __launch_bounds__(512) void dinv_kernel(float* X, int64_t n, int64_t ld, int64_t stride,
-                                                  const double* dinv64, int64_t dstride) {
+                                                  const double* tiles, int64_t dstride) {
     const int64_t k0 = (int64_t)blockIdx.x * NB;
-    const double* packed = dinv64 + (int64_t)blockIdx.y * dstride + (int64_t)blockIdx.x * NB * NB;
+    const double* packed = tiles + (int64_t)blockIdx.y * dstride + (int64_t)blockIdx.x * NB * NB;
     float* P = X + (int64_t)blockIdx.y * stride + k0 * ld + k0;
     const int nb = (int)std::min<int64_t>(NB, n - k0), lane = threadIdx.x & 63;
     switch (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {
@@ -729,16 +729,14 @@ __global__ void lower_to_upper_kernel(float* H, int64_t n, int64_t ld, int64_t s
     }
 }
 
-int64_t dinv_floats(int64_t batch, int64_t n) { return batch * cdiv(n, NB) * NB * NB; }
+int64_t tile_doubles(int64_t batch, int64_t n) { return batch * cdiv(n, NB) * NB * NB; }
 
-// fp64 copy of the Dinv blocks: after the fp32 ones, 256-byte aligned.
-double* dinv64_of(float* dinv, int64_t batch, int64_t n) {
-    const uintptr_t p = reinterpret_cast<uintptr_t>(dinv + dinv_floats(batch, n));
-    return reinterpret_cast<double*>((p + 255) & ~(uintptr_t)255);
+double* tiles_at(void* p) {
+    return reinterpret_cast<double*>((reinterpret_cast<uintptr_t>(p) + 255) & ~(uintptr_t)255);
 }
 
 // Lower Cholesky in place of `batch` matrices [n, n] (pitch ld, stride sH);
-// dinv64 receives every block's packed tiles (batch x nblk x NB x NB doubles).
+// tiles receives every block's packed tiles (batch x nblk x NB x NB doubles).
 //
 // Two-level right-looking: columns are taken in super-blocks of up to
 // SUPER_NB columns.  After each block's panel, only the rest of the
@@ -767,7 +765,7 @@ constexpr int64_t PANEL_GROUPS = 512;   // two work-groups per CU
 constexpr int64_t SPLIT_SEG = 2048;
 constexpr int64_t SPLIT_SYRK_BLOCKS = 15;
 
-int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* dinv64, int* info, hipStream_t st,
+int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* tiles, int* info, hipStream_t st,
           const SplitPlanes* Lp, bool merges) {
     const int64_t nblk = cdiv(n, NB);
     const int64_t dstride = nblk * NB * NB;
@@ -781,20 +779,20 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
         for (int64_t k0 = s0; k0 < s1; k0 += NB) {
             const int64_t kb = k0 / NB;
             const int nb = (int)std::min<int64_t>(NB, n - k0);
-            double* Dk64 = dinv64 + kb * NB * NB;
+            double* packed = tiles + kb * NB * NB;
             {
                 double fl = batch * (2.0 / 3.0) * nb * nb * nb, by = batch * 3.0 * 4 * nb * nb;
                 if (rest_pending) fl += rest.algo_flops, by += 4.0 * batch * (2.0 * rest.M * rest.K + 2.0 * rest.M * rest.N);
                 ProfScope prof_scope(st, PT_DIAG, fl, by);
                 const dim3 gd((unsigned)rest_tiles, 1, (unsigned)batch), wg(DIAG_WAVES * 64);
                 if (rest_pending && aligned)
-                    hipLaunchKernelGGL((potrf_diag_rest_kernel<true>), gd, wg, 0, st, H, ld, sH, k0, nb, Dk64, dstride,
+                    hipLaunchKernelGGL((potrf_diag_rest_kernel<true>), gd, wg, 0, st, H, ld, sH, k0, nb, packed, dstride,
                                        info, rest);
                 else if (rest_pending)
-                    hipLaunchKernelGGL((potrf_diag_rest_kernel<false>), gd, wg, 0, st, H, ld, sH, k0, nb, Dk64, dstride,
+                    hipLaunchKernelGGL((potrf_diag_rest_kernel<false>), gd, wg, 0, st, H, ld, sH, k0, nb, packed, dstride,
                                        info, rest);
                 else
-                    hipLaunchKernelGGL(potrf_diag_kernel, dim3((unsigned)batch), wg, 0, st, H, ld, sH, k0, nb, Dk64,
+                    hipLaunchKernelGGL(potrf_diag_kernel, dim3((unsigned)batch), wg, 0, st, H, ld, sH, k0, nb, packed,
                                        dstride, info);
                 IC_CHECK_LAUNCH();
                 rest_pending = false;
@@ -811,10 +809,10 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
                 const int groups = (int)cdiv(sets, PANEL_GROUPS);
                 const dim3 gd((unsigned)cdiv(sets, groups), (unsigned)batch);
                 if (aligned)
-                    hipLaunchKernelGGL((panel_solve_kernel<true>), gd, dim3(256), 0, st, A21, m, ld, sH, Dk64, dstride,
+                    hipLaunchKernelGGL((panel_solve_kernel<true>), gd, dim3(256), 0, st, A21, m, ld, sH, packed, dstride,
                                        groups);
                 else
-                    hipLaunchKernelGGL((panel_solve_kernel<false>), gd, dim3(256), 0, st, A21, m, ld, sH, Dk64, dstride,
+                    hipLaunchKernelGGL((panel_solve_kernel<false>), gd, dim3(256), 0, st, A21, m, ld, sH, packed, dstride,
                                        groups);
                 IC_CHECK_LAUNCH();
             }
@@ -866,9 +864,9 @@ int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* di
 }
 
 // X = L^-1 (lower triangle and the 128x128 diagonal blocks exact; the rest
-// of the upper triangle is scratch) from L (lower, in H) and the Dinv
-// blocks.  The diagonal blocks of X are the Dinv_k; then adjacent diagonal
-// inverses are merged level by level,
+// of the upper triangle is scratch) from L (lower, in H) and the diagonal
+// blocks' packed tiles, of which dinv_kernel forms X's diagonal blocks; then
+// adjacent diagonal inverses are merged level by level,
 //     [L11 0; L21 L22]^-1 = [X11 0; X21 X22],   X21 = -X22 (L21 X11),
 // with T (or T^T when the halves differ in size) parked in the unused
 // upper block of the merged square.  All pairs of one level that have the same shape run as one
@@ -963,11 +961,11 @@ static int merge_pairs_split(float* X, int64_t n, int64_t ld, int64_t r0, int64_
     return IC_OK;
 }
 
-int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_t sH, const double* dinv64,
+int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_t sH, const double* tiles,
           hipStream_t st, const SplitWork* w) {
     const int64_t nblk = cdiv(n, NB);
     const int64_t dstride = nblk * NB * NB;
-    hipLaunchKernelGGL(dinv_kernel, dim3((unsigned)nblk, (unsigned)batch), dim3(512), 0, st, X, n, ld, sH, dinv64,
+    hipLaunchKernelGGL(dinv_kernel, dim3((unsigned)nblk, (unsigned)batch), dim3(512), 0, st, X, n, ld, sH, tiles,
                        dstride);
     IC_CHECK_LAUNCH();
     // segments of rows [start, start + len); merged pairwise per level
@@ -1046,8 +1044,7 @@ static int64_t split_batch(int64_t batch, int64_t n, int64_t room) {
 }
 
 extern "C" int64_t ic_hessian_inverse_min_workspace_bytes(int64_t batch, int64_t n) {
-    return (batch * n * n + dinv_floats(batch, n)) * (int64_t)sizeof(float) +
-           dinv_floats(batch, n) * (int64_t)sizeof(double) + 256;
+    return batch * n * n * (int64_t)sizeof(float) + tile_doubles(batch, n) * (int64_t)sizeof(double) + 256;
 }
 
 extern "C" int64_t ic_hessian_inverse_workspace_bytes(int64_t batch, int64_t n) {
@@ -1058,13 +1055,13 @@ extern "C" int64_t ic_hessian_inverse_workspace_bytes(int64_t batch, int64_t n) 
 
 // `batch` damped matrices H -> their inverses (ic_hessian_inverse's methods);
 // X: batch n^2 floats.
-static int inverse(float* H, int64_t batch, int64_t n, int method, int* info, int* info2, float* X, double* dinv64,
+static int inverse(float* H, int64_t batch, int64_t n, int method, int* info, int* info2, float* X, double* tiles,
                    const SplitWork* w, hipStream_t st) {
     const int64_t ld = n, sH = n * n;
     const SplitPlanes* Lp = w ? &w->L : nullptr;
-    int rc = potrf(H, batch, n, ld, sH, dinv64, info, st, Lp, true);
+    int rc = potrf(H, batch, n, ld, sH, tiles, info, st, Lp, true);
     if (rc) return rc;
-    rc = trtri(H, X, batch, n, ld, sH, dinv64, st, w);
+    rc = trtri(H, X, batch, n, ld, sH, tiles, st, w);
     if (rc) return rc;
     // H^-1 (upper triangle incl. diagonal) = X^T X  -> H
     const double flops = (double)batch * 2.0 * (double)n * (n + 1) * (n + 2) / 6.0;
@@ -1085,7 +1082,7 @@ static int inverse(float* H, int64_t batch, int64_t n, int method, int* info, in
     if ((rc = mirror_upper(H, batch, n, ld, sH, st))) return rc;
     if (method == 1) {
         // upper Cholesky factor of H^-1 (converter/gptq.py:91-110): L2 = chol(H^-1), return L2^T
-        rc = potrf(H, batch, n, ld, sH, dinv64, info2, st, Lp, false);
+        rc = potrf(H, batch, n, ld, sH, tiles, info2, st, Lp, false);
         if (rc) return rc;
         dim3 tb(16, 16), tg((unsigned)cdiv(n, 16), (unsigned)cdiv(n, 16), (unsigned)batch);
         hipLaunchKernelGGL(lower_to_upper_kernel, tg, tb, 0, st, H, n, ld, sH);
@@ -1106,21 +1103,20 @@ extern "C" int ic_hessian_inverse_sized(float* H, int64_t batch, int64_t n, floa
     hipStream_t st = as_stream(stream);
     const int64_t sH = n * n;
     float* X = reinterpret_cast<float*>(workspace);
-    float* dinv = X + batch * sH;
-    double* dinv64 = dinv64_of(dinv, batch, n);
+    double* tiles = tiles_at(X + batch * sH);
     IC_CHECK_HIP(hipMemsetAsync(info, 0, batch * sizeof(int), st));
     hipLaunchKernelGGL(damp_kernel, dim3((unsigned)batch), dim3(256), 0, st, H, n, n, sH, damping);
     IC_CHECK_LAUNCH();
     const int64_t step = split_batch(batch, n, workspace_bytes - least);
-    if (step <= 0) return inverse(H, batch, n, method, info, info + batch, X, dinv64, nullptr, st);
-    const uintptr_t end = reinterpret_cast<uintptr_t>(dinv64 + dinv_floats(batch, n));
+    if (step <= 0) return inverse(H, batch, n, method, info, info + batch, X, tiles, nullptr, st);
+    const uintptr_t end = reinterpret_cast<uintptr_t>(tiles + tile_doubles(batch, n));
     char* planes = reinterpret_cast<char*>((end + 255) & ~(uintptr_t)255);
     for (int64_t b = 0; b < batch; b += step) {
         const int64_t m = std::min(step, batch - b);
         SplitWork w;
         split_bytes(m, n, planes, &w);
         int rc = inverse(H + b * sH, m, n, method, info + b, info + batch + b, X + b * sH,
-                         dinv64 + dinv_floats(b, n), &w, st);
+                         tiles + tile_doubles(b, n), &w, st);
         if (rc) return rc;
     }
     return IC_OK;
@@ -1160,7 +1156,6 @@ extern "C" int ic_cholesky(float* H, int64_t batch, int64_t n, int* info, void* 
     if (n == 0 || batch == 0) return IC_OK;
     hipStream_t st = as_stream(stream);
     IC_CHECK_HIP(hipMemsetAsync(info, 0, batch * sizeof(int), st));
-    float* dinv = reinterpret_cast<float*>(workspace) + batch * n * n;
-    double* dinv64 = dinv64_of(dinv, batch, n);
-    return potrf(H, batch, n, n, n * n, dinv64, info, st);
+    double* tiles = tiles_at(reinterpret_cast<float*>(workspace) + batch * n * n);
+    return potrf(H, batch, n, n, n * n, tiles, info, st);
 }

@@ -7,10 +7,10 @@
 
 namespace icq {
 
-// floats of a workspace region for `batch` matrices of order n; the fp64
-// Dinv blocks follow it at dinv64_of(dinv, batch, n).
-int64_t dinv_floats(int64_t batch, int64_t n);
-double* dinv64_of(float* dinv, int64_t batch, int64_t n);
+// potrf's fp64 tiles of the diagonal blocks (packed as chol.hip describes) for
+// `batch` matrices of order n: their doubles, and their place from p on.
+int64_t tile_doubles(int64_t batch, int64_t n);
+double* tiles_at(void* p);
 
 // Lower Cholesky in place of `batch` matrices [n, n] (pitch ld, stride sH);
 // info[b] receives the 1-based column of the first non-positive pivot (or
@@ -19,7 +19,7 @@ double* dinv64_of(float* dinv, int64_t batch, int64_t n);
 // Lp: planes for L (SP_LOWER): the larger trailing updates are split products,
 // and with `merges` the planes then hold the blocks that trtri's split merges
 // read.
-int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* dinv64, int* info, hipStream_t st,
+int potrf(float* H, int64_t batch, int64_t n, int64_t ld, int64_t sH, double* tiles, int* info, hipStream_t st,
           const SplitPlanes* Lp = nullptr, bool merges = false);
 
 // Split planes of a large inverse: L (from potrf), X^T (whole on return), X
@@ -28,10 +28,10 @@ struct SplitWork {
     SplitPlanes L, XT, XR, T;
 };
 
-// X = L^-1 from potrf's L and fp64 Dinv blocks (rounded to fp32 on the
-// diagonal of X): the lower triangle of X is exact, its strict upper
+// X = L^-1 from potrf's L and tiles (the diagonal blocks inverted in fp64 and
+// rounded to fp32): the lower triangle of X is exact, its strict upper
 // triangle outside the diagonal blocks is scratch.
-int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_t sH, const double* dinv64,
+int trtri(const float* L, float* X, int64_t batch, int64_t n, int64_t ld, int64_t sH, const double* tiles,
           hipStream_t st, const SplitWork* w = nullptr);
 
 }  // namespace icq

@@ -484,8 +484,8 @@ static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Workspace carve-up (every piece 256-byte aligned).
 struct LrWork {
-    float *Y, *Q, *G, *X, *dinv, *T, *Vs, *x, *y, *Gp;
-    double *dinv64, *A0, *A1, *V, *U, *part, *scal;
+    float *Y, *Q, *G, *X, *T, *Vs, *x, *y, *Gp;
+    double *tiles, *A0, *A1, *V, *U, *part, *scal;
     int *info, *rank;
 };
 
@@ -511,7 +511,7 @@ static size_t lr_layout(int64_t n, int64_t p, char* base, LrWork* w) {
     t.x = (float*)take((size_t)n * 4);
     t.Gp = (float*)take((size_t)GRAM_SPLIT * pp4);
     t.y = (float*)take((size_t)n * 4);
-    t.dinv = (float*)take((size_t)dinv_floats(1, p) * 4 + (size_t)dinv_floats(1, p) * 8 + 512);
+    t.tiles = (double*)take((size_t)tile_doubles(1, p) * 8);
     t.A0 = (double*)take(pp8);
     t.A1 = (double*)take(pp8);
     t.V = (double*)take(pp8);
@@ -520,10 +520,7 @@ static size_t lr_layout(int64_t n, int64_t p, char* base, LrWork* w) {
     t.part = (double*)take((size_t)LR_PARTS * 2 * 8);
     t.scal = (double*)take(8 * 8);
     t.info = (int*)take(64);
-    if (base) {
-        t.dinv64 = dinv64_of(t.dinv, 1, p);
-        *w = t;
-    }
+    if (base) *w = t;
     return off + 256;
 }
 
@@ -568,8 +565,8 @@ static int cholqr_pass(const float* Y, float* Q, int64_t n, int64_t p, float shi
         hipLaunchKernelGGL(shift_diag_kernel, dim3(1), dim3(256), 0, st, w.G, p, shift_rel);
         IC_CHECK_LAUNCH();
     }
-    if ((rc = potrf(w.G, 1, p, p, p * p, w.dinv64, w.info, st))) return rc;
-    if ((rc = trtri(w.G, w.X, 1, p, p, p * p, w.dinv64, st))) return rc;
+    if ((rc = potrf(w.G, 1, p, p, p * p, w.tiles, w.info, st))) return rc;
+    if ((rc = trtri(w.G, w.X, 1, p, p, p * p, w.tiles, st))) return rc;
     hipLaunchKernelGGL(zero_upper_kernel, dim3(egrid_lr(p * p)), dim3(256), 0, st, w.X, p);
     IC_CHECK_LAUNCH();
     // Q = Y X^T  (X = L^-1 lower, so op(B) = X^T is upper triangular)
@@ -656,7 +653,7 @@ extern "C" int ic_lowrank_eigs(const float* H, int64_t n, int64_t p, int iters, 
                                (double)refuse_rel);
             IC_CHECK_LAUNCH();
             int* test_info = w.info + 1 + (it - test_lo);
-            if ((rc = potrf(w.T, 1, p, p, p * p, w.dinv64, test_info, st))) return rc;
+            if ((rc = potrf(w.T, 1, p, p, p * p, w.tiles, test_info, st))) return rc;
             int pd_info = 0;
             IC_CHECK_HIP(hipMemcpyAsync(&pd_info, test_info, sizeof(int), hipMemcpyDeviceToHost, st));
             IC_CHECK_HIP(hipStreamSynchronize(st));
