@@ -78,6 +78,26 @@ def test_eigs_subspace_planted(gpu_dev):
         assert r.abs().max().item() <= 2e-5 * 50.0
 
 
+@pytest.mark.parametrize("n,p,decades", [(600, 244, 5.0), (600, 244, 3.0), (1024, 372, 4.0), (1500, 514, 4.0)])
+def test_eigs_subspace_without_gap(gpu_dev, n, p, decades):
+    """p < n, a log-spaced spectrum: no gap behind the kept pairs.  After 8
+    steps of H + mu I (mu = 1e-3 lambda_max) the share of eigenvector j > p in
+    the basis' i-th direction has shrunk by ((l_j + mu) / (l_i + mu))^8, from a
+    random start of about sqrt(n / p) at most; its square moves eigenvalue i
+    down by that part of l_i.  The bound below is that for each i, beside
+    fp32's 1e-5 of the largest."""
+    evs = torch.logspace(0.0, -decades, n, dtype=torch.float64)
+    H = _planted(n, evs, n)
+    ev, U, _ = _eigs(H, p, 8, gpu_dev)
+    want = torch.linalg.eigvalsh(H.double()).flip(0)
+    share = ((want[p] + 1e-3) / (want[:p] + 1e-3)) ** 8 * n / (p ** 0.5)
+    low = want[:p] - ev.double()
+    assert (low >= -1e-5).all(), low.min().item()          # Ritz values do not exceed the eigenvalues
+    bound = (1e-5 + want[:p] * share.clamp(max=1.0) ** 2)
+    assert (low <= bound).all(), (low / bound).max().item()
+    assert (U.double().T @ U.double() - torch.eye(p, dtype=torch.float64)).abs().max().item() < 1e-5
+
+
 def test_lowrank_decompose_decisions(gpu_dev):
     """Rank count and both refusal gates, against the oracle's eigh."""
     from int_crush_converter_amd.greedy import lowrank_decompose
