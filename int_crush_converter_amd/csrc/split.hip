@@ -1,10 +1,11 @@
 // Products of fp32 matrices as six bf16 MFMA products of split operands, and
 // the kernels that split them (layout and terms: split.hpp).
 //
-// Bound by the matrix cores' power: v_mfma_f32_32x32x16_bf16 reaches 2.47
-// PFLOP/s on zeros and 1.71 on random operands here (a sixth of which is the
-// fp32 rate), and the 12288 inverse's products keep it 70-79 % busy at the
-// clock that leaves.  Against v_mfma_f32_16x16x4_f32 (gemm_dev.hpp) on the
+// Bound by the matrix cores' power: a loop of v_mfma_f32_32x32x16_bf16 on
+// registers reaches 2.48 PFLOP/s on zeros and 1.94 on uniform random operands
+// (a sixth of which is the fp32 rate), and the 12288 inverse keeps the matrix
+// cores 71 % busy in its merges and X^T X, 55 % in its K = 1024 updates, at
+// the clock that leaves.  Against v_mfma_f32_16x16x4_f32 (gemm_dev.hpp) on the
 // 12288 x 12288 inverse: X^T X 4.99 -> 3.58 ms (173 TFLOP/s of fp32 work),
 // K = 1024 update of 11264 rows 1.14 -> 0.67 ms (196), merge T = L21 X11 of
 // 4096 x 8192 1.69 -> 1.30 ms (211); the inverse 20.9 -> 16.1 ms.  Its error
