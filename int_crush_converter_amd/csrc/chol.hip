@@ -1031,7 +1031,12 @@ static int64_t split_bytes(int64_t batch, int64_t n, char* base, SplitWork* w) {
 constexpr int64_t SPLIT_MAX_N = 65536, SPLIT_MAX_BYTES = 64LL << 30;
 // Up to SPLIT_ALIGNED_N the fp32 kernels keep up where their rows are aligned
 // (a layer with a 3072 x 3072 Hessian 4.03 ms, 4.08 split); where they are not
-// they do not (2901, Cholesky method: 4.13 ms, 4.05 split).
+// they do not (2901, Cholesky method: 4.13 ms, 4.05 split).  Around both lines
+// the two are as fast and the split products are more precise, so that they
+// begin where they cost 1.4 % at most.  Inverses, split over fp32 products: not
+// aligned 2049 1.003, 2301 1.008, 2501 0.984, 2701 0.964, 3071 0.925; aligned
+// 3076 0.908, 3136 1.014, 3200 1.005, 3456 1.004, 3584 0.997, 3840 0.976, 4096
+// 0.967, 5120 0.918.
 constexpr int64_t SPLIT_ALIGNED_N = 3072;
 static bool splits(int64_t n) {
     return n > (n % 4 == 0 ? SPLIT_ALIGNED_N : SPLIT_SEG) && n <= SPLIT_MAX_N;
