@@ -48,19 +48,19 @@ WORKLOADS = {
     "gptq_int4_dlr128_rot256_4096x12288": ("dlr", 4096, 12288, {"rank": 128}),
     # GPTQ INT4 with PiSO scales (128 coarse + 16 fine candidates per row) on the headline layer
     "gptq_int4_piso_rot256_4096x12288": ("piso", 4096, 12288, {"samples": 8192, "cpu_rows": 512}),
-    # configs[4] end to end, file to file (quantize_model with streaming I/O):
-    # the first 4 of its 40 DiT blocks, bf16 safetensors + 3-D calibration
+    # a 40-block DiT end to end, file to file (quantize_model with streaming I/O):
+    # its first 4 blocks, bf16 safetensors + 3-D calibration
     "e2e_dit_gptq_int4_rot256_4blocks": ("e2e", 0, 0, {"blocks": 4, "samples": 4096,
                                                        "layers": [("attn.qkv", 12288, 4096), ("attn.proj", 4096, 4096),
                                                                   ("mlp.up", 16384, 4096),
                                                                   ("mlp.down", 4096, 16384)]}),
-    # configs[4] end to end at its stated size: all 40 DiT blocks (16 GB of bf16
+    # the same at its full size: all 40 DiT blocks (16 GB of bf16
     # weights in, 4 GB of packed codes out), file to file
     "e2e_dit_gptq_int4_rot256_40blocks": ("e2e", 0, 0, {"blocks": 40, "samples": 4096,
                                                         "layers": [("attn.qkv", 12288, 4096), ("attn.proj", 4096, 4096),
                                                                    ("mlp.up", 16384, 4096),
                                                                    ("mlp.down", 4096, 16384)]}),
-    # one block of configs[4]'s 40-block DiT sweep: four layers, block-diagonal Hessians
+    # one block of the 40-block DiT: four layers, block-diagonal Hessians
     "gptq_int4_rot256_dit_block": ("dit", 0, 0, {"layers": [("qkv", 12288, 4096), ("proj", 4096, 4096),
                                                             ("mlp_up", 16384, 4096), ("mlp_down", 4096, 16384)],
                                                  "samples": 4096}),
@@ -81,7 +81,7 @@ def block_hessian(X):
 
 
 def make_e2e_files(extra, seed=0):
-    """A model file with configs[4]'s layer shapes (bf16, N(0, 0.02^2)) and a
+    """A model file with the DiT's layer shapes (bf16, N(0, 0.02^2)) and a
     calibration file of 3-D block-diagonal Hessians, in a temporary folder."""
     import tempfile
     import torch
@@ -137,7 +137,7 @@ def make_inputs(kind, M, N, extra, seed=0):
         cols = torch.randperm(N, generator=g, device=dev)[: max(1, N // 100)]
         W[:, cols] *= 20
     if kind == "ldlq":
-        # Student-t(4) scaled to std 0.02 (configs[3]); t = z / sqrt(chi2_4 / 4)
+        # Student-t(4) scaled to std 0.02; t = z / sqrt(chi2_4 / 4)
         z = torch.randn(M, N, generator=g, device=dev)
         chi = (torch.randn(M, N, 4, generator=g, device=dev) ** 2).sum(-1)
         W = z / torch.sqrt(chi / 4) * (0.02 / math.sqrt(2))
@@ -409,7 +409,7 @@ def roofline_from(prof, workload):
 
 def hbm_ceiling(nbytes=1 << 30, reps=10):
     """GB/s of the library's streaming probes (ic_hbm_stream) on 1 GiB: the
-    practical HBM ceiling of the box for each read/write mix.  Bytes counted:
+    practical HBM ceiling of the machine for each read/write mix.  Bytes counted:
     copy read + written, read, write, convert 2 read + 4 written per element."""
     import torch
     from int_crush_converter_amd import _native as nat
@@ -534,7 +534,7 @@ def main():
                             for k, v in prof.items() if v["launches"]}
     if not args.no_cpu_baseline:
         # torch's intra-op threads: OMP_NUM_THREADS, the CPU share of one GPU
-        # on the box (os.cpu_count() counts the whole host)
+        # on the machine (os.cpu_count() counts the whole host)
         threads = torch.get_num_threads()
         log(f"[bench] CPU baseline (oracle, {threads} threads): 1 layer")
         if kind == "dit":
@@ -568,7 +568,7 @@ def main():
 
 
 def main_e2e(args, extra):
-    """File to file: quantize_model on a synthetic slice of configs[4]; a step
+    """File to file: quantize_model on a synthetic slice of the DiT; a step
     is one whole conversion.  Also times the reference's load-all /
     save-once I/O on the same files (in_memory_ms)."""
     import shutil

@@ -5,7 +5,7 @@ CPU only).
 ``libicq.so`` whose host code (argument checks, error strings, launch
 set-up, the loader's view of the exports) is compiled with AddressSanitizer
 and whose device code is built as usual, then runs ``tests/test_abi.py``
-against it with the sanitizer runtime preloaded.  The GPU box never builds
+against it with the sanitizer runtime preloaded.  No GPU machine builds
 or loads this variant.
 """
 

@@ -1,4 +1,4 @@
-// Streaming kernels that measure the HBM ceiling of the box the library runs
+// Streaming kernels that measure the HBM ceiling of the machine the library runs
 // on (bench.py --hbm-ceiling): the bandwidth the path's HBM-bound kernels
 // are compared with.  Every access is a 16-byte vector, consecutive lanes
 // touch consecutive 16-byte words, and each thread keeps four loads in

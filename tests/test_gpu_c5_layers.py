@@ -1,4 +1,4 @@
-"""GPU parity at configs[4]'s real layer shapes: GPTQ INT4 rot256 with a
+"""GPU parity at the 40-block DiT's real layer shapes: GPTQ INT4 rot256 with a
 block-diagonal calibration Hessian [in/256, 256, 256] (each block X^T X / 4096
 of a seeded X with LogNormal(0, 1) channel scales), bf16 weights N(0, 0.02^2),
 for the DiT block's widest layers: qkv [12288, 4096] (16 groups) and

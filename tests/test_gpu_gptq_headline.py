@@ -1,4 +1,4 @@
-"""North-star parity at the benchmark's own layer shapes: GPTQ INT4 rot256,
+"""Parity at the benchmark's own layer shapes: GPTQ INT4 rot256,
 block 128, damping 0.01, on the bench recipe (bf16 W ~ N(0, 0.02^2),
 H = X^T X / 8192 with LogNormal(0, 1) channel scales) at [4096, 12288]
 (the metric's layer) and C3's [3072, 12288] and [12288, 3072].
@@ -12,7 +12,7 @@ algorithm, converter/rounding.py:37-103 and converter/gptq.py:113-121,
   and the lazy update subtracts one 128-column block's product at a time
   (each summed in k order from zero, as MKL's sgemm does at K = 128), so
   the codes are expected bit-exact (measured: all equal at every shape); the
-  assertion is the north-star bar, >= 99.9 % of codes equal and
+  assertion is the stated bar, >= 99.9 % of codes equal and
   tr(dW H dW^T) within 1e-3 relative.
 * full path: the GPU computes its own damped inverse.  GPTQ feeds every
   rounding forward, so the bar is relative to the reference's own noise on

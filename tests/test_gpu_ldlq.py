@@ -258,7 +258,7 @@ def _student_t(M, N, g):
 
 @pytest.mark.parametrize("n", [1024, 2048])
 def test_ldlq_c4_shaped_vs_reference_noise(gpu_dev, n):
-    """configs[3]'s recipe at M = N = n: Student-t (nu = 4) weights scaled to
+    """The LDLQ benchmark's recipe at M = N = n: Student-t (nu = 4) weights scaled to
     std 0.02, rot256, weight-only H = W^T W / M, 2 LDLQ iterations, then 5
     greedy passes through the default dispatch (eigen-truncation, refused by
     the rank gate for this full-rank H, then the full-rank search), against
@@ -323,11 +323,11 @@ def test_ldlq_c4_shaped_vs_reference_noise(gpu_dev, n):
 
 
 def test_ldlq_c4_full_size_vs_reference_noise(gpu_dev):
-    """configs[3] at its real size, M = N = 4096 (one of its 8 layers):
+    """The LDLQ benchmark at its real size, M = N = 4096 (one of its 8 layers):
     the same recipe and bars as the test above, with the oracle's noise
     taken from the one alternative that changes both summation orders
     (a two-half W^T W and half the CPU threads), to bound the CPU time.
-    The scale bar is stated against that noise; north-star's literal bar is
+    The scale bar is stated against that noise; the literal bar is
     1 fp16 ulp, and the measured maximum is printed beside it."""
     from int_crush_converter_amd.ldlq import ldlq_quantize_layer
     n = 4096
